@@ -327,3 +327,48 @@ def test_backward_project_adam_equals_separate_steps(gpu, cfg, render_deg):
     np.testing.assert_array_equal(stats[2][0], stats[0][0])
     np.testing.assert_array_equal(stats[2][1], stats[0][1])
     assert (stats[0][1] != stats[1][1]).sum() > 100   # the separate statistics counted Gaussians
+
+
+@pytest.mark.parametrize("deg", [0, 1, 2, 3])
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 1025])
+@pytest.mark.parametrize("kind", ["mixed", "all pruned", "all densified", "unaligned"])
+def test_adc_apply_blocks_bit_exact(gpu, oracle, n, deg, kind):
+    """Compaction at the edges of a workgroup's 256 old Gaussians, for every SH degree, with runs of
+    no new slot, of two per Gaussian, and with SH and moments at addresses no wide access may use."""
+    from tdgs_amd import training
+    g = _random_scene(n, deg, 7)
+    rng = np.random.default_rng(8)
+    adc_h = oracle.AdcHost(n)
+    adc_h.accum[:] = 1.0 if kind == "all densified" else np.abs(rng.normal(0, 3e-4, n)).astype(np.float32)
+    adc_h.counts[:] = 1
+    prune = {"all pruned": 1e9, "all densified": -1e9}.get(kind, float(host.logit32(0.1)))
+    args = (prune, False, 0.0, 2e-4, float(np.log(np.float32(0.06))))
+    nn = oracle.adc_plan(adc_h, g, *args)
+    assert {"all pruned": nn == 0, "all densified": nn == 2 * n}.get(kind, True)
+    adam_h = oracle.AdamHost(n, deg, [1e-3] * 6)
+    for arr in (adam_h.means, adam_h.opacity, adam_h.scaling, adam_h.rotation, adam_h.sh):
+        arr[...] = rng.normal(size=arr.shape).astype(np.float32)
+    gd = gpu.TrainableGaussiansVector.from_host(g, 0)
+    opt = training.AdamOptimizer(gd, training.TrainingOptions())
+
+    def on_device(a):
+        off = 1 if kind == "unaligned" else 0
+        t = torch.empty(a.size + off, dtype=torch.float32, device=DEV)[off:].view(a.shape)
+        t.copy_(torch.from_numpy(a))
+        return t
+
+    gd.sh = on_device(g.sh)
+    for name in ("means", "opacity", "scaling", "sh"):
+        setattr(opt.moments, name, on_device(getattr(adam_h, name)))
+    opt.moments.rotation.copy_(torch.from_numpy(adam_h.rotation))
+    adc = training.AdaptiveDensityControlBuffers(n, 0)
+    for dst, src in ((adc.prune, adc_h.prune), (adc.densify, adc_h.densify), (adc.clone, adc_h.clone), (adc.cs, adc_h.cs)):
+        dst.copy_(torch.from_numpy(src))
+    log_split = float(np.log(np.float32(1 / 1.6)))
+    got = training.adaptive_density_control_(adc, gd, opt, nn, log_split, 42).to_host()
+    ng_h, nm_h = oracle.adc_apply(adc_h, g, adam_h, log_split, 42)
+    for a, b in ((got.means_opacity, ng_h.means_opacity), (got.scaling, ng_h.scaling),
+                 (got.rotation, ng_h.rotation), (got.sh, ng_h.sh)):
+        np.testing.assert_array_equal(a, b)
+    for name in ("means", "opacity", "scaling", "rotation", "sh"):
+        np.testing.assert_array_equal(getattr(opt.moments, name).cpu().numpy(), getattr(nm_h, name))

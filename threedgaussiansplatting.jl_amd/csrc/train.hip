@@ -202,75 +202,122 @@ struct AdcApplyArgs {
     const uint8_t* clone;
     const int32_t* cs;
     int64_t n;
-    int h;
     float log_split;
     uint64_t seed;
 };
 
-__device__ __forceinline__ void copy_block(const float* s, float* d, int count) {
-    for (int k = 0; k < count; ++k) d[k] = s[k];
+constexpr int kAdcThreads = 256;
+constexpr int kAdcUnroll = 4;
+
+// Copies the rows (ROW floats each) of nslots consecutive new slots from their old Gaussians:
+// slot j takes row s_slot[j] >> 1 of src, or zeros when MOMENTS and bit 0 of s_slot[j] is clear; a
+// slot with a negative s_slot[j] is left as it is.
+// Thread t moves items t, t + kAdcThreads, ... of V floats, so loads and stores run along the
+// rows; kAdcUnroll loads are issued before their stores (which could alias the next loads).
+template <int ROW, int V, bool MOMENTS>
+__device__ __forceinline__ void adc_copy_rows_v(const float* __restrict__ src, float* __restrict__ dst,
+                                                const int16_t* s_slot, int nslots) {
+    typedef float Vec __attribute__((ext_vector_type(V)));
+    constexpr int Q = ROW / V;
+    const int items = nslots * Q;
+    for (int base = threadIdx.x; base < items; base += kAdcUnroll * kAdcThreads) {
+        Vec v[kAdcUnroll];
+        int e[kAdcUnroll];
+#pragma unroll
+        for (int u = 0; u < kAdcUnroll; ++u) {
+            const int k = base + kAdcThreads * u, j = k / Q;
+            v[u] = Vec(0.0f);
+            e[u] = k < items ? s_slot[j] : -1;
+            if (e[u] >= 0 && (!MOMENTS || (e[u] & 1)))
+                v[u] = reinterpret_cast<const Vec*>(src)[(e[u] >> 1) * Q + (k - j * Q)];
+        }
+#pragma unroll
+        for (int u = 0; u < kAdcUnroll; ++u)
+            if (e[u] >= 0) reinterpret_cast<Vec*>(dst)[base + kAdcThreads * u] = v[u];
+    }
 }
-__device__ __forceinline__ void zero_block(float* d, int count) {
-    for (int k = 0; k < count; ++k) d[k] = 0.0f;
+
+// The widest item that divides a row; single floats where an array is not aligned to it.
+template <int ROW, bool MOMENTS>
+__device__ __forceinline__ void adc_copy_rows(const float* src, float* dst, int64_t row_src, int64_t row_dst,
+                                              const int16_t* s_slot, int nslots) {
+    constexpr int V = ROW % 4 == 0 ? 4 : ROW % 2 == 0 ? 2 : 1;
+    const bool aligned = ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & (4 * V - 1)) == 0;
+    src += ROW * row_src;
+    dst += ROW * row_dst;
+    if (V == 1 || aligned) adc_copy_rows_v<ROW, V, MOMENTS>(src, dst, s_slot, nslots);
+    else adc_copy_rows_v<ROW, 1, MOMENTS>(src, dst, s_slot, nslots);
 }
 
 // fill_means_opacity_features_adc_kernel!, fill_scaling_features_adc_kernel! (gaussians.jl
 // :1589-1694), the indexlastaxis gathers (:1563-1571) and fill_adam_moments_component_kernel!
-// (optimizer.jl:1342-1378), fused: one thread per old Gaussian writes all its new slots.
-__global__ __launch_bounds__(256) void k_adc_apply(AdcApplyArgs a) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= a.n || a.prune[i]) return;
-    const int h = a.h;
-    const int64_t last = (int64_t)a.cs[i] - 1;
-    const bool dens = a.densify[i], cl = a.clone[i];
-    const int64_t first = dens ? last - 1 : last;
-    const float4 mo = reinterpret_cast<const float4*>(a.src.means_opacity)[i];
-    const float s0 = a.src.scaling[3 * i], s1 = a.src.scaling[3 * i + 1], s2 = a.src.scaling[3 * i + 2];
-    const float4 q = reinterpret_cast<const float4*>(a.src.rotation)[i];
-    float z[6] = {0, 0, 0, 0, 0, 0};
-    float R[9];
-    float sc[3];
-    const bool split = dens && !cl;
-    if (split) {
-        quat_to_rot(q.x, q.y, q.z, q.w, R);
-        sc[0] = exp_f(s0); sc[1] = exp_f(s1); sc[2] = exp_f(s2);
-        normal_pair(a.seed, (uint64_t)i, 0, &z[0], &z[1]);
-        normal_pair(a.seed, (uint64_t)i, 1, &z[2], &z[3]);
-        normal_pair(a.seed, (uint64_t)i, 2, &z[4], &z[5]);
-    }
-    for (int64_t ni = first; ni <= last; ++ni) {
-        const int j = (int)(ni - first);
-        float4 nm = mo;
-        float ns0 = s0, ns1 = s1, ns2 = s2;
+// (optimizer.jl:1342-1378), fused. A workgroup takes kAdcThreads consecutive old Gaussians, whose
+// new slots (at most two each) are one contiguous run: the threads write their Gaussians' means,
+// scalings and rotations and note each slot's source in LDS, then the workgroup copies the
+// spherical harmonics and the moments along the run. Bound by HBM: 708 B in and out per
+// Gaussian at SH3. (One thread per Gaussian copying its own blocks moved them in 4-byte words 192
+// and 384 bytes apart: @OLD@ us at 500k Gaussians, SH3, 8% densified, against @NEW@ us.)
+template <int H>
+__global__ __launch_bounds__(kAdcThreads) void k_adc_apply(AdcApplyArgs a) {
+    __shared__ int16_t s_slot[2 * kAdcThreads];   // (local old Gaussian << 1) | its moments are kept
+    __shared__ int64_t s_run[2];                  // the run of new slots: first, past the last
+    const int t = threadIdx.x;
+    const int64_t i0 = (int64_t)blockIdx.x * kAdcThreads, i = i0 + t;
+    const bool valid = i < a.n;
+    const bool pr = !valid || a.prune[i], dens = !pr && a.densify[i], cl = dens && a.clone[i];
+    const int64_t past = valid ? a.cs[i] : 0;
+    const int item = (pr ? 0 : 1) + (dens ? 1 : 0);
+    s_slot[t] = s_slot[t + kAdcThreads] = -1;
+    if (t == 0) s_run[0] = past - (a.prune[i] ? 0 : 1) - (a.densify[i] ? 1 : 0);
+    if (valid && (t == kAdcThreads - 1 || i == a.n - 1)) s_run[1] = past;
+    __syncthreads();
+    const int64_t run = s_run[0];
+    const int64_t span = s_run[1] - run;
+    const int nslots = span < 0 ? 0 : span > 2 * kAdcThreads ? 2 * kAdcThreads : (int)span;
+    if (item > 0) {
+        const int64_t first = past - item;
+        const float4 mo = reinterpret_cast<const float4*>(a.src.means_opacity)[i];
+        const float s0 = a.src.scaling[3 * i], s1 = a.src.scaling[3 * i + 1], s2 = a.src.scaling[3 * i + 2];
+        const float4 q = reinterpret_cast<const float4*>(a.src.rotation)[i];
+        float z[6] = {0, 0, 0, 0, 0, 0};
+        float R[9];
+        float sc[3];
+        const bool split = dens && !cl;
         if (split) {
-            const float w0 = z[3 * j] * sc[0], w1 = z[3 * j + 1] * sc[1], w2 = z[3 * j + 2] * sc[2];
-            nm.x = mo.x + fmaf(R[2], w2, fmaf(R[1], w1, R[0] * w0));
-            nm.y = mo.y + fmaf(R[5], w2, fmaf(R[4], w1, R[3] * w0));
-            nm.z = mo.z + fmaf(R[8], w2, fmaf(R[7], w1, R[6] * w0));
-            ns0 = s0 + a.log_split; ns1 = s1 + a.log_split; ns2 = s2 + a.log_split;
+            quat_to_rot(q.x, q.y, q.z, q.w, R);
+            sc[0] = exp_f(s0); sc[1] = exp_f(s1); sc[2] = exp_f(s2);
+            normal_pair(a.seed, (uint64_t)i, 0, &z[0], &z[1]);
+            normal_pair(a.seed, (uint64_t)i, 1, &z[2], &z[3]);
+            normal_pair(a.seed, (uint64_t)i, 2, &z[4], &z[5]);
         }
-        reinterpret_cast<float4*>(a.dst.means_opacity)[ni] = nm;
-        a.dst.scaling[3 * ni] = ns0;
-        a.dst.scaling[3 * ni + 1] = ns1;
-        a.dst.scaling[3 * ni + 2] = ns2;
-        reinterpret_cast<float4*>(a.dst.rotation)[ni] = q;
-        copy_block(a.src.sh + (int64_t)3 * h * i, a.dst.sh + (int64_t)3 * h * ni, 3 * h);
-        // moments: carried over and first clone keep theirs, second clone and splits start at 0
-        const bool keep_m = !dens || (cl && ni == first);
-        if (keep_m) {
-            copy_block(a.sm.means_moments + 6 * i, a.dm.means_moments + 6 * ni, 6);
-            copy_block(a.sm.opacity_moments + 2 * i, a.dm.opacity_moments + 2 * ni, 2);
-            copy_block(a.sm.scaling_moments + 6 * i, a.dm.scaling_moments + 6 * ni, 6);
-            copy_block(a.sm.rotation_moments + 8 * i, a.dm.rotation_moments + 8 * ni, 8);
-            copy_block(a.sm.sh_moments + (int64_t)6 * h * i, a.dm.sh_moments + (int64_t)6 * h * ni, 6 * h);
-        } else {
-            zero_block(a.dm.means_moments + 6 * ni, 6);
-            zero_block(a.dm.opacity_moments + 2 * ni, 2);
-            zero_block(a.dm.scaling_moments + 6 * ni, 6);
-            zero_block(a.dm.rotation_moments + 8 * ni, 8);
-            zero_block(a.dm.sh_moments + (int64_t)6 * h * ni, 6 * h);
+        for (int j = 0; j < item; ++j) {
+            const int64_t ni = first + j;
+            float4 nm = mo;
+            float ns0 = s0, ns1 = s1, ns2 = s2;
+            if (split) {
+                const float w0 = z[3 * j] * sc[0], w1 = z[3 * j + 1] * sc[1], w2 = z[3 * j + 2] * sc[2];
+                nm.x = mo.x + fmaf(R[2], w2, fmaf(R[1], w1, R[0] * w0));
+                nm.y = mo.y + fmaf(R[5], w2, fmaf(R[4], w1, R[3] * w0));
+                nm.z = mo.z + fmaf(R[8], w2, fmaf(R[7], w1, R[6] * w0));
+                ns0 = s0 + a.log_split; ns1 = s1 + a.log_split; ns2 = s2 + a.log_split;
+            }
+            reinterpret_cast<float4*>(a.dst.means_opacity)[ni] = nm;
+            a.dst.scaling[3 * ni] = ns0;
+            a.dst.scaling[3 * ni + 1] = ns1;
+            a.dst.scaling[3 * ni + 2] = ns2;
+            reinterpret_cast<float4*>(a.dst.rotation)[ni] = q;
+            // moments: carried over and first clone keep theirs, second clone and splits start at 0
+            const bool keep_m = !dens || (cl && j == 0);
+            if (ni >= run && ni - run < 2 * kAdcThreads) s_slot[ni - run] = (int16_t)(2 * t + (keep_m ? 1 : 0));
         }
     }
+    __syncthreads();
+    adc_copy_rows<3 * H, false>(a.src.sh, a.dst.sh, i0, run, s_slot, nslots);
+    adc_copy_rows<6, true>(a.sm.means_moments, a.dm.means_moments, i0, run, s_slot, nslots);
+    adc_copy_rows<2, true>(a.sm.opacity_moments, a.dm.opacity_moments, i0, run, s_slot, nslots);
+    adc_copy_rows<6, true>(a.sm.scaling_moments, a.dm.scaling_moments, i0, run, s_slot, nslots);
+    adc_copy_rows<8, true>(a.sm.rotation_moments, a.dm.rotation_moments, i0, run, s_slot, nslots);
+    adc_copy_rows<6 * H, true>(a.sm.sh_moments, a.dm.sh_moments, i0, run, s_slot, nslots);
 }
 
 // adjust_fgidx_to_gidx_adc_kernel! (training.jl:514-541).
@@ -484,10 +531,13 @@ int tdgs_adc_apply(void* stream, const tdgs_adc_buffers* adc, const tdgs_gaussia
     a.src = *src; a.dst = *dst; a.sm = *src_m; a.dm = *dst_m;
     a.prune = adc->prune; a.densify = adc->densify; a.clone = adc->clone; a.cs = adc->new_counts_cs;
     a.n = src->n;
-    a.h = (src->sh_degree + 1) * (src->sh_degree + 1);
     a.log_split = log_split_factor;
     a.seed = seed;
-    k_adc_apply<<<(unsigned)ceil_div(src->n, 256), 256, 0, s>>>(a);
+    const unsigned grid = (unsigned)ceil_div(src->n, kAdcThreads);
+    if (src->sh_degree == 0) k_adc_apply<1><<<grid, kAdcThreads, 0, s>>>(a);
+    else if (src->sh_degree == 1) k_adc_apply<4><<<grid, kAdcThreads, 0, s>>>(a);
+    else if (src->sh_degree == 2) k_adc_apply<9><<<grid, kAdcThreads, 0, s>>>(a);
+    else k_adc_apply<16><<<grid, kAdcThreads, 0, s>>>(a);
     TDGS_LAUNCHED();
     return TDGS_OK;
 }

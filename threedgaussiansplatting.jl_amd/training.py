@@ -84,17 +84,19 @@ def annealed_means_lr(iteration_nb: int, options: TrainingOptions) -> float:
 
 
 class GaussianAdamMomentsLearningRatesVector:
-    """Adam moments (m1, m2 interleaved) and learning rates (optimizer.jl:9-195)."""
+    """Adam moments (m1, m2 interleaved) and learning rates (optimizer.jl:9-195). zero=False
+    leaves the moments uninitialised, for a caller that writes every one."""
 
-    def __init__(self, n, sh_degree, lrs, device=0):
+    def __init__(self, n, sh_degree, lrs, device=0, zero=True):
         d = _dev(device)
         h = (sh_degree + 1) ** 2
+        new = torch.zeros if zero else torch.empty
         self.sh_degree = int(sh_degree)
-        self.means = torch.zeros((n, 3, 2), dtype=torch.float32, device=d)
-        self.opacity = torch.zeros((n, 2), dtype=torch.float32, device=d)
-        self.scaling = torch.zeros((n, 3, 2), dtype=torch.float32, device=d)
-        self.rotation = torch.zeros((n, 4, 2), dtype=torch.float32, device=d)
-        self.sh = torch.zeros((n, 3, h, 2), dtype=torch.float32, device=d)
+        self.means = new((n, 3, 2), dtype=torch.float32, device=d)
+        self.opacity = new((n, 2), dtype=torch.float32, device=d)
+        self.scaling = new((n, 3, 2), dtype=torch.float32, device=d)
+        self.rotation = new((n, 4, 2), dtype=torch.float32, device=d)
+        self.sh = new((n, 3, h, 2), dtype=torch.float32, device=d)
         (self.means_lr, self.opacity_lr, self.scaling_lr, self.rotation_lr, self.sh_dc_lr,
          self.sh_rest_lr) = [float(v) for v in lrs]
 
@@ -245,7 +247,8 @@ def adaptive_density_control_(adc, gaussians: TrainableGaussiansVector, optimize
                                    torch.empty((n_new, 4), dtype=torch.float32, device=dev),
                                    torch.empty((n_new, 3, h), dtype=torch.float32, device=dev))
     old_m = optimizer.moments
-    new_m = GaussianAdamMomentsLearningRatesVector(n_new, gaussians.sh_degree, old_m.lrs(), dev.index)
+    new_m = GaussianAdamMomentsLearningRatesVector(n_new, gaussians.sh_degree, old_m.lrs(), dev.index,
+                                                   zero=False)   # (tdgs_adc_apply writes every slot)
     src_m, dst_m = optimizer.struct(), None
     optimizer.moments = new_m
     dst_m = optimizer.struct()
