@@ -156,3 +156,65 @@ def test_backward_tiny_min_alpha_takes_range_checked_path(gpu, oracle):
     got, ref = _run(gpu, oracle, w.gaussians, cam, t, opts, rand_grad)
     for k in ["grads2d"] + ARRAYS:
         assert rel_l2(got[k], ref[k]) <= REL_L2, (k, rel_l2(got[k], ref[k]))
+
+
+@pytest.mark.parametrize("w,h,tile", [
+    # one, two and four pixels per lane (by the image's number of 8 x 8 blocks and the tile's size)
+    (330, 250, (16, 16)), (330, 250, (16, 32)), (330, 250, (10, 12)), (330, 250, (16, 8)), (330, 250, (8, 8)),
+    (655, 636, (16, 16)), (655, 636, (16, 32)), (655, 636, (24, 8)), (655, 636, (13, 20)),
+    (813, 797, (16, 16)), (813, 797, (16, 32)), (813, 797, (32, 32)), (813, 797, (13, 20)), (813, 797, (16, 8)),
+    (813, 797, (8, 8))])
+@pytest.mark.parametrize("scene", ["usual", "needles"])
+def test_backward_by_image_size(gpu, oracle, w, h, tile, scene):
+    """Each split of a tile's pixels over lanes, blocks and wavefronts, ragged images, with usual
+    Gaussians and with needles (axis ratios to 400), whose boxes decide what a block looks at. (Of the
+    needles the 2D gradients are compared, which the blending computes: their chain to the scales
+    multiplies float32 rounding by the inverse of a nearly singular covariance, twice.)"""
+    wl = synthetic.config(0, n=1500)
+    g = wl.gaussians
+    rng = np.random.default_rng(3)
+    if scene == "needles":
+        g.scaling[:] = rng.uniform(-6.0, 0.0, g.scaling.shape).astype(np.float32)
+    cam = host.look_at_camera(w, h, 60.0, (0.0, 0.0, -4.0))
+    t = host.Tiling.for_camera(cam, *tile)
+    opts = host.RenderOptions.for_camera(cam, 0, background_color=(0.2, 0.1, 0.3))
+    gen = torch.Generator(device="cuda").manual_seed(17)
+
+    def rand_grad(rgb):
+        return (torch.rand(rgb.shape, generator=gen, device=rgb.device) - 0.5) * 1e-3
+
+    got, ref = _run(gpu, oracle, g, cam, t, opts, rand_grad)
+    for k in ["grads2d"] + (ARRAYS if scene == "usual" else []):
+        assert rel_l2(got[k], ref[k]) <= REL_L2, (k, rel_l2(got[k], ref[k]))
+
+
+@pytest.mark.parametrize("size", [640, 816])
+def test_backward_list_lengths_at_chunk_and_batch_ends_of_large_images(gpu, oracle, size):
+    """Lists of 1 to 3 records past a chunk of 64 and a batch of 128 with two and four pixels per lane."""
+    cam = host.look_at_camera(size, size, 60.0, (0.0, 0.0, -4.0))
+    t = host.Tiling.for_camera(cam, 16, 16)
+    opts = host.RenderOptions.for_camera(cam, 0, background_color=(0.2, 0.1, 0.3))
+    gen = torch.Generator(device="cuda").manual_seed(5)
+
+    def rand_grad(rgb):
+        return (torch.rand(rgb.shape, generator=gen, device=rgb.device) - 0.5) * 1e-3
+
+    for k in (1, 63, 65, 127, 129, 131):
+        got, ref = _run(gpu, oracle, stacked_faint_gaussians(k), cam, t, opts, rand_grad)
+        for name in ["grads2d"] + ARRAYS:
+            assert rel_l2(got[name], ref[name]) <= REL_L2, (k, name, rel_l2(got[name], ref[name]))
+
+
+def test_backward_no_alpha_in_range(gpu):
+    """max_alpha below min_alpha: nothing contributes, every gradient is zero."""
+    wl = synthetic.config(0, n=500)
+    cam = wl.cameras[0]
+    t = host.Tiling.for_camera(cam, 16, 16)
+    opts = host.RenderOptions.for_camera(cam, 0, min_alpha=0.01, max_alpha=0.005)
+    g = gpu.TrainableGaussiansVector.from_host(wl.gaussians, 0)
+    out = gpu.RenderOutputs.for_camera(cam, 0)
+    buf = gpu.RenderBuffers(len(g), t, 0)
+    gpu.render_(out, g, cam, t, opts, buf)
+    fg = gpu.FilteredGaussiansGradientsVector(buf.capacity, 0, 0)
+    gpu.backward_(fg, torch.ones_like(out.rgb), out, g, cam, t, opts, buf)
+    assert buf.nb_keys > 0 and float(fg.grads2d.abs().max()) == 0.0 and int(out.last.max()) == 0

@@ -4,7 +4,7 @@
 // Reference: src/backward_core.jl:37-452 (+ helpers :465-964), src/backward_structs.jl:250-257.
 //
 // Backward blending (backward_render_tiles_kernel!, :96-293): one workgroup per tile, one
-// thread per four pixels. The reference lets every pixel start at its own last contributor and
+// thread per four pixels (two or one on images too small to fill the chip). The reference lets every pixel start at its own last contributor and
 // issues 9 float atomics per (pixel, Gaussian) pair. Here the wavefront walks the tile's
 // sorted list back to front in lock step (a lane whose last contributor lies before the
 // current entry contributes zero), so every pixel meets its entries in the reference's order;
@@ -42,37 +42,79 @@ __device__ __forceinline__ float halve_swap16(float x, float y) {
     return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, hi);
 }
 
+// x[i] = (x[i] + y[i]) halved at lane distance 8 or 4 (D): lanes whose bit D is clear get x[i] summed
+// with lane ^ D's x[i], the others y[i] with lane ^ D's y[i]. A DPP add writes only the lanes of the
+// 4-lane banks its bank_mask names and leaves the others, so each half is one add with the rotation
+// that reaches its partner (row_ror:n reads lane - n of the row) and no select: 8.4 issue cycles a
+// pair, against 10.5 for two selects and a DPP add and 11 for a permlane swap and an add (measured
+// at eight wavefronts per SIMD). A DPP read, or a permlane swap, needs two wait states after the
+// write of its register, which the compiler does not see inside the block: hence the s_nop around it.
+template <int D>
+__device__ __forceinline__ void halve_dpp(float (&x)[8], const float (&y)[8]) {
+#define TDGS_HALF(I, CTRL, BANKS) "v_add_f32_dpp %" #I ", %" #I ", %" #I " " CTRL " row_mask:0xf bank_mask:" BANKS "\n"
+#define TDGS_OTHER(I, J, CTRL, BANKS) "v_add_f32_dpp %" #I ", %" #J ", %" #J " " CTRL " row_mask:0xf bank_mask:" BANKS "\n"
+#define TDGS_HALVE(CX, BX, CY, BY)                                                                          \
+    asm("s_nop 1\n" TDGS_HALF(0, CX, BX) TDGS_HALF(1, CX, BX) TDGS_HALF(2, CX, BX) TDGS_HALF(3, CX, BX)       \
+            TDGS_HALF(4, CX, BX) TDGS_HALF(5, CX, BX) TDGS_HALF(6, CX, BX) TDGS_HALF(7, CX, BX)               \
+                TDGS_OTHER(0, 8, CY, BY) TDGS_OTHER(1, 9, CY, BY) TDGS_OTHER(2, 10, CY, BY)                   \
+                    TDGS_OTHER(3, 11, CY, BY) TDGS_OTHER(4, 12, CY, BY) TDGS_OTHER(5, 13, CY, BY)             \
+                        TDGS_OTHER(6, 14, CY, BY) TDGS_OTHER(7, 15, CY, BY) "s_nop 1"                        \
+        : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7])      \
+        : "v"(y[0]), "v"(y[1]), "v"(y[2]), "v"(y[3]), "v"(y[4]), "v"(y[5]), "v"(y[6]), "v"(y[7]))
+    static_assert(D == 8 || D == 4, "a distance inside a row, of whole banks");
+    if constexpr (D == 8) TDGS_HALVE("row_ror:8", "0x3", "row_ror:8", "0xc");
+    else TDGS_HALVE("row_ror:12", "0x5", "row_ror:4", "0xa");
+#undef TDGS_HALVE
+#undef TDGS_OTHER
+#undef TDGS_HALF
+}
+
 // Sums 64 values per lane over the wavefront by recursive halving: at the step of lane
 // distance D each lane keeps the half of its values whose index has the lane's bit D,
-// adds the partner lane's copy of that half and passes on the other half. Six steps
-// (D = 32, 16 by permlane swaps; 8, 4, 2, 1 by DPP inside a row) and 63 adds in total leave
-// in lane l the wavefront sum of v[l]. v is destroyed.
+// adds the partner lane's copy of that half and passes on the other half. Six steps, the
+// cheapest on the most values (8 and 4 by masked DPP adds: 48 of the 63 sums; then 32 and 16 by
+// permlane swaps, 2 and 1 by selects and DPP), leave in lane l the wavefront sum of v[l]. v is
+// destroyed.
 __device__ __forceinline__ float wave_transpose_sum64(float (&v)[64]) {
     const int lane = __lane_id();
+    // value index i = 16 r + 8 d3 + 4 d2 + c: the pairs (i, i + 8), eight of them at a time
 #pragma unroll
-    for (int i = 0; i < 32; ++i) v[i] = halve_swap32(v[i], v[i + 32]);
+    for (int r = 0; r < 4; ++r) {
+        float x[8], y[8];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) v[i] = halve_swap16(v[i], v[i + 16]);
-    const bool b3 = lane & 8, b2 = lane & 4, b1 = lane & 2, b0 = lane & 1;
+        for (int k = 0; k < 8; ++k) {
+            x[k] = v[16 * r + k];
+            y[k] = v[16 * r + 8 + k];
+        }
+        halve_dpp<8>(x, y);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const float send = b3 ? v[i] : v[i + 8], keep = b3 ? v[i + 8] : v[i];
-        v[i] = keep + dpp_f32<0x128>(send);                       // row_ror:8 = lane ^ 8
+        for (int k = 0; k < 8; ++k) v[16 * r + k] = x[k];
     }
+    // the pairs (i, i + 4) of two r at a time
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float send = b2 ? v[i] : v[i + 4], keep = b2 ? v[i + 4] : v[i];
-        // lane ^ 4 by ds_swizzle in bit-mask mode (and 0x1f, xor 4). One unconditional
-        // cross-lane read: a select between two DPP rotations gets turned into a branch, and
-        // a DPP read from a lane switched off by that branch returns 0.
-        v[i] = keep + __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, send), 0x101f));
+    for (int r = 0; r < 4; r += 2) {
+        float x[8], y[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            x[k] = v[16 * (r + k / 4) + k % 4];
+            y[k] = v[16 * (r + k / 4) + 4 + k % 4];
+        }
+        halve_dpp<4>(x, y);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[16 * (r + k / 4) + k % 4] = x[k];
     }
+    float w[8];   // w[4 h + c]: index 16 h + c, h = 0, 1 (after the distance 32)
+#pragma unroll
+    for (int k = 0; k < 8; ++k) w[k] = halve_swap32(v[16 * (k / 4) + k % 4], v[16 * (k / 4) + 32 + k % 4]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) w[k] = halve_swap16(w[k], w[k + 4]);
+    const bool b1 = lane & 2, b0 = lane & 1;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const float send = b1 ? v[i] : v[i + 2], keep = b1 ? v[i + 2] : v[i];
-        v[i] = keep + dpp_f32<0x4e>(send);                        // quad_perm [2,3,0,1]
+        const float send = b1 ? w[i] : w[i + 2], keep = b1 ? w[i + 2] : w[i];
+        w[i] = keep + dpp_f32<0x4e>(send);                        // quad_perm [2,3,0,1]
     }
-    const float send = b0 ? v[0] : v[1], keep = b0 ? v[1] : v[0];
+    const float send = b0 ? w[0] : w[1], keep = b0 ? w[1] : w[0];
     return keep + dpp_f32<0xb1>(send);                            // quad_perm [1,0,3,2]
 }
 
@@ -134,13 +176,31 @@ struct __align__(16) BackRec {
     float4 a;  // mu_x mu_y A B
     float4 b;  // C cut a r     (cut: x below which a * G < min_alpha)
     float4 c;  // g b f M11     (f: the Gaussian's index, for the flush)
-    float4 d;  // M21 M22 - -
+    float4 d;  // M21 M22 r_x r_y
 };
+
+// The half sides (r_x, r_y) of a box around the mean outside which x < cut, for x = -(p du^2 + q du dv +
+// s dv^2) with p, s > 0: x = cut is an ellipse whose du reaches sqrt(-cut s / (p s - q^2 / 4)). The
+// determinant in double (p s and q^2 / 4 agree to 1 in 1e4 and more for needles), the box widened by
+// 1e-4 of its size and 1e-2 pixels for the rounding of x, the cut and the square root; no bound
+// (infinite sides) where the form is not definite or anything is NaN, none at all (negative
+// sides) where a positive cut says that no alpha reaches min_alpha. The cut's own margin (1e-3) covers its error.
+__device__ __forceinline__ void cut_box(float A, float B, float C, float cut, float* rx, float* ry) {
+    const float p = -A, s = -C;
+    const double det = (double)p * s - 0.25 * (double)B * B;
+    const float k = -cut / (float)det;
+    const float x2 = k * s, y2 = k * p;
+    const bool bounded = p > 0.0f && s > 0.0f && det > 0.0 && x2 >= 0.0f && y2 >= 0.0f && x2 < kInf && y2 < kInf;
+    *rx = bounded ? fmaf(sqrtf(x2), 1.0001f, 0.01f) : kInf;
+    *ry = bounded ? fmaf(sqrtf(y2), 1.0001f, 0.01f) : kInf;
+    if (cut > 1e-3f) *rx = *ry = -kInf;
+}
 
 struct BackBlendArgs {
     int32_t W, H, TW, TH, ntx;
     float bg0, bg1, bg2, min_alpha, max_alpha;
     float log_min_alpha;   // log(min_alpha) - 1e-3 (-inf without a positive min_alpha)
+    int32_t batch;         // entries per batch, at most one per thread
     int64_t m;
     const int32_t* tiles_end;
     const int32_t* sorted_f;
@@ -154,31 +214,58 @@ struct BackBlendArgs {
 // SEP: the 2D gradients are the reference's four arrays (component addresses by select);
 // otherwise the interleaved 9 x capacity array (base[0] + 9 f + k).
 // PX pixels per lane: lane l of wavefront w takes pixels 64 PX w + 64 p + l, p < PX, of the
-// tile (NB = blockDim.x = NT / PX rounded up to whole wavefronts; a pixel index past NT is
+// tile (blockDim.x = NT / PX rounded up to whole wavefronts; a pixel index past NT is
 // off), so the per-entry record reads, votes, slot bookkeeping and transpose-sum serve 64 PX
 // pixels per wavefront; with tiles of 8 x 8 pixel blocks a wavefront holds PX consecutive
-// blocks. A batch holds NB entries. Four pixels per lane at four wavefronts per SIMD (128
-// VGPRs; a few per-batch values go to scratch) measured 345 us against 378 us for two pixels
-// per lane at 1M Gaussians, 1080p (three wavefronts per SIMD at 142 VGPRs: 365 us).
-constexpr int kBackPx = 4;
+// blocks. 128 VGPRs, four wavefronts per SIMD, so 4096 fill the chip.
+//
+// Where they do not, a wavefront walks its list nearly alone on its SIMD and the longest list's
+// walk is the kernel's time: one instruction after the other, ~850 cycles an entry at four pixels
+// per lane. Fewer pixels per lane mean more wavefronts with less work per entry, and a block that
+// fewer entries reach: with CULL a batch's entries are first tested, one per lane, by their boxes
+// against each slot's block, and the walk visits only those that reach it. The work grows (the
+// sums over the wavefront serve fewer pixels), so the filled chip keeps four pixels per lane, where
+// CULL's branches per slot cost more than the dead slots they skip (368 against 314 us at the
+// last line below). us, by 64-pixel blocks of the image, and image, Gaussians, tiles:
+//                                             PX = 4       2       1   (always 4 and every entry walked)
+//     520   200x150     3k  16x16               76.2    45.3    28.5   (76.4)
+//    1024   256x256    10k  16x16              178.3   105.7    63.4   (177.9)
+//    2500   400x400    20k  16x16              213.7   133.5    84.5   (211.8)
+//    4800   640x480   500k  16x16              298.4   203.4   177.8   (289.6)
+//    5776   600x600    60k  16x16              179.7   128.0   112.4   (174.8)
+//    8928   979x546    60k  16x32               93.9    59.2    64.3   (91.5)
+//   10000   800x800   200k  16x16              161.1   171.9   171.2   (162.3)
+//   17384   1297x840  500k  16x16              252.6   265.6   295.8   (259.3)
+//   32640   1920x1080   1M  16x16              324.1   371.7   440.8   (329.6)
+// Tiles of at most 64 PX / 2 pixels would leave half the lanes off (8 x 8 tiles, 800x600, 200k:
+// 180.6, 165.5, 143.2).
+constexpr int64_t kBackWaves1 = 6144, kBackWaves2 = 9216;   // blocks up to which PX is 1, 2
+constexpr int kBackBatch = 128;       // entries per batch with PX < 4, at most (64: 5% slower; 256: the same)
+constexpr size_t kBackLds = 56 << 10; // LDS of a workgroup, at most
 // BPC > 0 (tile sides multiples of 8, BPC = TH / 8 blocks of 8 x 8 pixels per block column,
 // BPC dividing PX): slot p's pixels are slot 0's moved by the constant (8 (p / BPC), 8 (p %
 // BPC)), so only slot 0's coordinates are kept per lane and the others' offsets from the
 // record are slot 0's plus a constant (three fewer register pairs: 323 us against 349 us at 1M
 // Gaussians, 1080p, where the loop's scratch spills went from 52 to 12 bytes per lane). The
 // subtraction order differs from the per-pixel form by rounding only. BPC = 0: any tile.
-template <bool SEP, int PX, int BPC>
-__global__ __launch_bounds__(1024 / kBackPx) __attribute__((amdgpu_waves_per_eu(4))) void k_backward_blend(
+//
+// What bounds the filled chip is VALU issue: ~75 instructions an entry (x of the four slots, compares,
+// 1.3 live slots' steps, a seventh of a transpose-sum), of which a multiply, add, FMA or move takes 2
+// cycles of a SIMD, a compare, select, DPP, integer or scalar-operand instruction about 4, exp2 and
+// reciprocal 8. Hence one compare per slot for the cut, the one for the last contributor only where
+// the cut leaves the slot, and the transpose-sum by masked DPP adds: 329.6 -> 324.1 us at 1M Gaussians, 1080p, 694 -> 688 us at 3M, 4K.
+template <bool SEP, int PX, int BPC, bool CULL>
+__global__ __launch_bounds__(1024 / PX) __attribute__((amdgpu_waves_per_eu(4))) void k_backward_blend(
     BackBlendArgs a) {
     extern __shared__ float4 s_raw4[];
     const int NT = a.TW * a.TH;
-    const int NB = (int)blockDim.x;
+    const int NTH = (int)blockDim.x, NB = a.batch;
     BackRec* s_rec = reinterpret_cast<BackRec*>(s_raw4);
     // Per-wavefront sums [wave][NB][9] (at most 4 wavefronts: 1024 / PX threads). A wavefront
     // takes each entry into at most one slot, so its transposed sums are plain stores (an LDS
     // atomic's round trip sat in front of the next entry's record reads); the flush adds the
     // wavefronts' copies.
-    const int NW = NB / kWave;
+    const int NW = NTH / kWave;
     float* s_acc = reinterpret_cast<float*>(s_rec + NB);
     float* s_accw = s_acc + (threadIdx.x / kWave) * (NB * 9);
     __shared__ int s_max_last;
@@ -222,7 +309,13 @@ __global__ __launch_bounds__(1024 / kBackPx) __attribute__((amdgpu_waves_per_eu(
         cu[p] = (float)U - 0.5f;
         cv[p] = (float)V - 0.5f;
     }
-    static_assert(BPC == 0 || PX % BPC == 0, "slot offsets are constant when BPC divides PX");
+    static_assert(BPC == 0 || PX % BPC == 0 || BPC % PX == 0, "constant slot offsets");
+    // The box of slot 0's pixel centres: corner (box_u, box_v), an 8 x 8 block, the others' moved as the
+    // slots are; the whole tile for every slot where the slots are no blocks (BPC = 0 but for PX = 1).
+    const bool blocks = BPC != 0 || (PX == 1 && ((a.TW | a.TH) & 7) == 0);
+    const int block0 = blocks ? __builtin_amdgcn_readfirstlane(t / kWave) * PX : 0;   // column-major
+    const int bpc = blocks ? a.TH >> 3 : 1;
+    const int box_u = (tx - 1) * a.TW + 8 * (block0 / bpc), box_v = (ty - 1) * a.TH + 8 * (block0 % bpc);
     const int slot = lane / 9, comp = lane - 9 * slot;
     const int partner = comp == 0 ? lane + 1 : comp == 1 ? lane - 1 : lane;
     const float scale = comp == 4 ? -1.0f : (comp == 3 || comp == 5) ? -0.5f : 1.0f;
@@ -232,7 +325,7 @@ __global__ __launch_bounds__(1024 / kBackPx) __attribute__((amdgpu_waves_per_eu(
     for (int p = 1; p < PX; ++p) lane_last = last[p] > lane_last ? last[p] : lane_last;
     const int wave_last = wave_max_i32(lane_last);
     if (t == 0) s_max_last = 0;
-    for (int k = t; k < NW * NB * 9; k += NB) s_acc[k] = 0.0f;
+    for (int k = t; k < NW * NB * 9; k += NTH) s_acc[k] = 0.0f;
     __syncthreads();
     if (lane == 0) atomicMax(&s_max_last, wave_last);
     __syncthreads();
@@ -261,7 +354,9 @@ __global__ __launch_bounds__(1024 / kBackPx) __attribute__((amdgpu_waves_per_eu(
             // of log_min_alpha; a NaN cut never skips)
             rec.b = make_float4(-0.5f * kLog2e * pr[5], kLog2e * (a.log_min_alpha - log_f(pr[2])), pr[2], pr[6]);
             rec.c = make_float4(pr[7], pr[8], __builtin_bit_cast(float, pf), pr[3]);
-            rec.d = make_float4(pr[4], pr[5], 0.0f, 0.0f);
+            float rx = 0.0f, ry = 0.0f;
+            if (CULL) cut_box(rec.a.z, rec.a.w, rec.b.x, rec.b.y, &rx, &ry);
+            rec.d = make_float4(pr[4], pr[5], rx, ry);
             s_rec[t] = rec;
         }
         __syncthreads();
@@ -271,86 +366,156 @@ __global__ __launch_bounds__(1024 / kBackPx) __attribute__((amdgpu_waves_per_eu(
         int last_rel[PX];
 #pragma unroll
         for (int p = 0; p < PX; ++p) last_rel[p] = (int)((int64_t)last[p] - lo);
+        const float max_alpha = a.max_alpha, min_alpha = a.min_alpha;
+        // One entry's step for the live lanes of pixel slot p, at exponent x and offset (du, dv).
+        auto step = [&](int p, uint64_t live, float x, float du, float dv, float alpha0, const float c[3], float* o) {
+            // G by the hardware base-2 exponential (v_exp_f32, ~1 ulp over the whole
+            // float range): the gradients are checked at relative L2, and the forward
+            // pass's bit-exact exp_f decides the contributors
+            const float G = __builtin_amdgcn_exp2f(x);
+            const float aG = alpha0 * G;
+            // min(aG, max_alpha) (v_min_f32: a NaN aG gives max_alpha)
+            float alpha;
+            asm("v_min_f32 %0, %1, %2" : "=v"(alpha) : "s"(max_alpha), "v"(aG));
+            // Branch-free: a lane that does not contribute runs the same steps with
+            // alpha = G = 0, so 1 / (1 - alpha) = 1 exactly and T, g . psi and the
+            // sums are left unchanged. (The contributors are decided by alpha, not by the cut alone:
+            // a cut rounded to float is off by up to 5e-7 of alpha, which on wide, faint Gaussians
+            // flips a pixel or two of each one's rim.)
+            const uint64_t cp = live & __builtin_amdgcn_ballot_w64(!(alpha < min_alpha));
+            float al, Gl;
+            asm("v_cndmask_b32 %0, 0, %1, %2" : "=v"(al) : "v"(alpha), "s"(cp));
+            asm("v_cndmask_b32 %0, 0, %1, %2" : "=v"(Gl) : "v"(G), "s"(cp));
+            backward_pair_sums(p == 0, al, __builtin_amdgcn_rcpf(1.0f - al), Gl, du, dv, c, g[p], &T[p], &gpsi[p], o);
+        };
+        // Offset of slot p's pixel from the entry's mean, the slot 0's (du0, dv0) moved by a constant.
+        auto offset = [&](int p, const float4& ra, float du0, float dv0, float* du, float* dv) {
+            *du = BPC == 0 ? cu[p] - ra.x : du0 + (float)(8 * (p / (BPC ? BPC : 1)));
+            *dv = BPC == 0 ? cv[p] - ra.y : dv0 + (float)(8 * (p % (BPC ? BPC : 1)));
+        };
+        // CULL: which entries of a 64-entry chunk reach which of the wavefront's pixel slots: lane l
+        // tests entry 64 ch + l's box against each slot's pixels, one vote per slot. The walk then
+        // visits only the entries and slots so found, by scalar bit scans.
+        uint64_t cand[PX], cand_any = 0;
+        auto vote = [&](int ch) {
+            const int e = 64 * ch + lane;
+            float mx = 0.0f, my = 0.0f, rx = -kInf, ry = -kInf;
+            if (e < jtop) {
+                const float2 m = *reinterpret_cast<const float2*>(&s_rec[e].a);
+                const float2 r = *reinterpret_cast<const float2*>(&s_rec[e].d.z);
+                mx = m.x; my = m.y; rx = r.x; ry = r.y;
+            }
+            cand_any = 0;
+            const float hu = blocks ? 3.5f : 0.5f * (float)a.TW, hv = blocks ? 3.5f : 0.5f * (float)a.TH;
+            const float ou = mx - ((float)box_u + 0.5f + hu), ov = my - ((float)box_v + 0.5f + hv);
+            const float wu = rx + hu, wv = ry + hv;
+#pragma unroll
+            for (int p = 0; p < PX; ++p) {
+                const bool hit = !(fabsf(ou - (float)(BPC ? 8 * (p / (BPC ? BPC : 1)) : 0)) > wu) &&
+                                 !(fabsf(ov - (float)(BPC ? 8 * (p % (BPC ? BPC : 1)) : 0)) > wv);
+                cand[p] = __builtin_amdgcn_ballot_w64(hit);
+                cand_any |= cand[p];
+            }
+        };
         // Entries back to front; the 9 contributions of up to kSlots consecutive contributing
         // entries are kept per lane and summed over the wavefront in one transpose-sum, after
         // which lane l holds component l % 9 of slot l / 9 and adds it to the tile's LDS sum.
-        int j = __builtin_amdgcn_readfirstlane(jtop - 1);   // wave-uniform: scalar loop control
-        // after a transpose-sum lane l holds component comp = l % 9 of slot l / 9
-        const float max_alpha = a.max_alpha;
-        while (j >= 0) {
+        // (wave-uniform: scalar loop control)
+        int j = __builtin_amdgcn_readfirstlane(jtop - 1);
+        int ch = __builtin_amdgcn_readfirstlane((jtop - 1) >> 6);   // CULL: the chunk; negative: no entry
+        if (CULL && ch >= 0) vote(ch);
+        while (CULL ? cand_any != 0 || ch > 0 : j >= 0) {
             float v[64];
             int js[kSlots];
 #pragma unroll
             for (int e = 0; e < kSlots; ++e) {
                 js[e] = -1;
                 float* o = v + 9 * e;
-                while (j >= 0) {
-                    const int jj = j--;
-                    const float4 ra = s_rec[jj].a, rb = s_rec[jj].b;
-                    const float2 rc = *reinterpret_cast<const float2*>(&s_rec[jj].c);
-                    float du[PX], dv[PX], x[PX];
-                    bool live[PX];
-                    uint64_t any[PX], any_all = 0;
+                // An entry takes a slot when some lane of the wavefront is live for it. A pixel slot
+                // no lane is live in is skipped as a whole (a wave-uniform branch): its steps would
+                // leave T, g . psi and the sums unchanged. When it is the first slot, the others
+                // add to zeroed sums. (An off pixel has last = 0, so jj < last_rel fails for it.)
+                if constexpr (CULL) {
+                    while (cand_any != 0) {
+                        const int jb = 63 - __builtin_clzll(cand_any);
+                        const uint64_t bit = 1ull << jb;
+                        cand_any &= ~bit;
+                        const int jj = 64 * ch + jb;
+                        const float4 ra = s_rec[jj].a, rb = s_rec[jj].b;
+                        const float2 rc = *reinterpret_cast<const float2*>(&s_rec[jj].c);
+                        const float c[3] = {rb.w, rc.x, rc.y};
+                        const float du0 = BPC == 0 ? 0.0f : cu[0] - ra.x, dv0 = BPC == 0 ? 0.0f : cv[0] - ra.y;
+                        bool taken = false;
 #pragma unroll
-                    for (int p = 0; p < PX; ++p) {
-                        if (BPC == 0 || p == 0) {
-                            du[p] = cu[p] - ra.x;
-                            dv[p] = cv[p] - ra.y;
-                        } else {
-                            // (tile_pixel's blocks w PX + p, column-major, BPC per column)
-                            du[p] = du[0] + (float)(8 * (p / (BPC > 0 ? BPC : 1)));
-                            dv[p] = dv[0] + (float)(8 * (p % (BPC > 0 ? BPC : 1)));
-                        }
-                        x[p] = fmaf(fmaf(ra.z, du[p], ra.w * dv[p]), du[p], rb.x * dv[p] * dv[p]);
-                        // (an off pixel has last = 0, so jj < last_rel fails for it)
-                        const bool before = jj < last_rel[p], above = !(x[p] < rb.y);
-                        live[p] = before & above;
-                        // the vote as masks of the two compares (the mask of their conjunction
-                        // takes two more instructions)
-                        any[p] = __builtin_amdgcn_ballot_w64(before) & __builtin_amdgcn_ballot_w64(above);
-                        any_all |= any[p];
-                    }
-                    if (any_all == 0) continue;
-                    const float c[3] = {rb.w, rc.x, rc.y};
-#pragma unroll
-                    for (int p = 0; p < PX; ++p) {
-                        // A pixel slot no lane of the wavefront is live in is skipped as a whole
-                        // (a wave-uniform branch): its steps would leave T, g . psi and the sums
-                        // unchanged. When it is the first slot, the others add to zeroed sums.
-                        if (any[p] == 0) {
-                            if (p == 0) {
-#pragma unroll
-                                for (int k = 0; k < 9; ++k) o[k] = 0.0f;
+                        for (int p = 0; p < PX; ++p) {
+                            uint64_t live = 0;   // lanes the entry may contribute to
+                            float du, dv, x;
+                            if (cand[p] & bit) {
+                                offset(p, ra, du0, dv0, &du, &dv);
+                                x = fmaf(fmaf(ra.z, du, ra.w * dv), du, rb.x * dv * dv);
+                                live = __builtin_amdgcn_ballot_w64(!(x < rb.y)) &
+                                       __builtin_amdgcn_ballot_w64(jj < last_rel[p]);
                             }
-                            continue;
+                            if (live == 0) {
+                                if (p == 0 && PX > 1) {
+#pragma unroll
+                                    for (int k = 0; k < 9; ++k) o[k] = 0.0f;
+                                }
+                                continue;
+                            }
+                            taken = true;
+                            step(p, live, x, du, dv, rb.z, c, o);
                         }
-                        // G by the hardware base-2 exponential (v_exp_f32, ~1 ulp over the whole
-                        // float range): the gradients are checked at relative L2, and the forward
-                        // pass's bit-exact exp_f decides the contributors
-                        const float G = __builtin_amdgcn_exp2f(x[p]);
-                        const float aG = rb.z * G;
-                        // min(aG, max_alpha) (v_min_f32: a NaN aG gives max_alpha)
-                        float alpha;
-                        asm("v_min_f32 %0, %1, %2" : "=v"(alpha) : "s"(max_alpha), "v"(aG));
-                        const bool cp = live[p] & !(alpha < a.min_alpha);
-                        // Branch-free: a lane that does not contribute runs the same steps with
-                        // alpha = G = 0, so 1 / (1 - alpha) = 1 exactly and T, g . psi and the
-                        // sums are left unchanged.
-                        const float al = cp ? alpha : 0.0f;
-                        backward_pair_sums(p == 0, al, __builtin_amdgcn_rcpf(1.0f - al), cp ? G : 0.0f, du[p], dv[p],
-                                           c, g[p], &T[p], &gpsi[p], o);
+                        if (taken) {
+                            js[e] = jj;
+                            break;
+                        }
                     }
-                    // The entry takes a slot when some lane of the wavefront is live for it (its
-                    // sums are zero if no lane's alpha reaches min_alpha after all).
-                    js[e] = __builtin_amdgcn_readfirstlane(jj);
-                    break;
+                } else {
+                    while (j >= 0) {
+                        const int jj = j--;
+                        const float4 ra = s_rec[jj].a, rb = s_rec[jj].b;
+                        const float2 rc = *reinterpret_cast<const float2*>(&s_rec[jj].c);
+                        const float du0 = BPC == 0 ? 0.0f : cu[0] - ra.x, dv0 = BPC == 0 ? 0.0f : cv[0] - ra.y;
+                        float du[PX], dv[PX], x[PX];
+                        uint64_t live[PX], any = 0;   // lanes the entry may contribute to
+#pragma unroll
+                        for (int p = 0; p < PX; ++p) {
+                            offset(p, ra, du0, dv0, &du[p], &dv[p]);
+                            x[p] = fmaf(fmaf(ra.z, du[p], ra.w * dv[p]), du[p], rb.x * dv[p] * dv[p]);
+                            live[p] = __builtin_amdgcn_ballot_w64(!(x[p] < rb.y));
+                        }
+                        // A compare costs the issue slots of two multiply-adds: the pixels' last
+                        // contributors are looked at only for the slots the entry reaches.
+#pragma unroll
+                        for (int p = 0; p < PX; ++p) {
+                            if (live[p] != 0) live[p] &= __builtin_amdgcn_ballot_w64(jj < last_rel[p]);
+                            any |= live[p];
+                        }
+                        if (any == 0) continue;
+                        const float c[3] = {rb.w, rc.x, rc.y};
+#pragma unroll
+                        for (int p = 0; p < PX; ++p) {
+                            if (live[p] == 0) {
+                                if (p == 0) {
+#pragma unroll
+                                    for (int k = 0; k < 9; ++k) o[k] = 0.0f;
+                                }
+                                continue;
+                            }
+                            step(p, live[p], x[p], du[p], dv[p], rb.z, c, o);
+                        }
+                        js[e] = __builtin_amdgcn_readfirstlane(jj);
+                        break;
+                    }
                 }
-                if (js[e] < 0) {   // a slot left empty at the end of the batch sums zeros
+                if (js[e] < 0) {   // a slot left empty at the end of a chunk sums zeros
 #pragma unroll
                     for (int k = 0; k < 9; ++k) o[k] = 0.0f;
                 }
             }
-            if (js[0] < 0) break;
+            if (CULL && cand_any == 0 && ch > 0) vote(--ch);
+            if (js[0] < 0) continue;
             v[63] = 0.0f;
             const float sum = wave_transpose_sum64(v);
             int jl = -1;
@@ -370,7 +535,7 @@ __global__ __launch_bounds__(1024 / kBackPx) __attribute__((amdgpu_waves_per_eu(
         // Flush with lane i on component i % 9 of entry i / 9: one atomic instruction covers
         // the 36-byte slots of ~7 Gaussians instead of one scattered word of 64. Each element
         // is cleared for the next batch by the thread that reads it.
-        for (int i = t; i < 9 * nb; i += NB) {
+        for (int i = t; i < 9 * nb; i += NTH) {
             int ii = i;
             asm volatile("" : "+v"(ii));   // (keeps the element index 32-bit: no 64-bit induction variables)
             float v = 0.0f;
@@ -817,25 +982,35 @@ int tdgs_backward_render_tiles(void* stream, tdgs_gradients* grads, const float*
     a.m = buf->key_capacity;
     a.tiles_end = buf->tiles_end; a.sorted_f = buf->sorted_values; a.f2d = buf->f2d;
     a.rgb_grad = rgb_grad; a.T = out->T; a.last = out->last; a.g2 = g2v;
-    // kBackPx pixels per thread, in whole wavefronts (the transpose-sum reads all 64 lanes;
-    // the pixels past the tile's are off)
-    const int nt = ((tiling->tile_width * tiling->tile_height + kBackPx - 1) / kBackPx + kWave - 1) / kWave * kWave;
-    const size_t lds = (size_t)nt * (sizeof(BackRec) + (size_t)(nt / kWave) * 9 * sizeof(float));
+    // px pixels per thread, in whole wavefronts (the transpose-sum reads all 64 lanes; the pixels
+    // past the tile's are off); see k_backward_blend for the choice.
+    const int pixels = tiling->tile_width * tiling->tile_height;
+    const int64_t blocks = (int64_t)tiling->nb_tiles_x * tiling->nb_tiles_y * ceil_div(pixels, kWave);
+    const int px = pixels <= kWave || blocks <= kBackWaves1 ? 1 : pixels <= 2 * kWave || blocks <= kBackWaves2 ? 2 : 4;
+    const int nt = (int)ceil_div(pixels, px * kWave) * kWave;
+    const int nw = nt / kWave;
+    a.batch = px == 4 || nt < kBackBatch ? nt : kBackBatch;
+    while (a.batch * (sizeof(BackRec) + nw * 9 * sizeof(float)) > kBackLds) a.batch /= 2;
+    const size_t lds = a.batch * (sizeof(BackRec) + nw * 9 * sizeof(float));
     const dim3 grid(tiling->nb_tiles_x, tiling->nb_tiles_y);
     // tiles of 8 x 8 pixel blocks with 1, 2 or 4 blocks per column take the constant slot offsets
     const int bpc = tiling->tile_width % 8 == 0 && tiling->tile_height % 8 == 0 ? tiling->tile_height / 8 : 0;
-#define TDGS_BB(SEP_, BPC_) k_backward_blend<SEP_, kBackPx, BPC_><<<grid, nt, lds, s>>>(a)
-    if (grads->grads2d) {
-        if (bpc == 1) TDGS_BB(false, 1);
-        else if (bpc == 2) TDGS_BB(false, 2);
-        else if (bpc == 4) TDGS_BB(false, 4);
-        else TDGS_BB(false, 0);
-    } else {
-        if (bpc == 1) TDGS_BB(true, 1);
-        else if (bpc == 2) TDGS_BB(true, 2);
-        else if (bpc == 4) TDGS_BB(true, 4);
-        else TDGS_BB(true, 0);
-    }
+#define TDGS_BB3(SEP_, PX_, BPC_) k_backward_blend<SEP_, PX_, BPC_, (PX_ < 4)><<<grid, nt, lds, s>>>(a)
+#define TDGS_BB2(PX_, BPC_)                              \
+    do {                                                 \
+        if (grads->grads2d) TDGS_BB3(false, PX_, BPC_);  \
+        else TDGS_BB3(true, PX_, BPC_);                  \
+    } while (0)
+#define TDGS_BB(BPC_)                        \
+    do {                                     \
+        if (px == 4) TDGS_BB2(4, BPC_);      \
+        else if (px == 2) TDGS_BB2(2, BPC_); \
+        else TDGS_BB2(1, 0);                 \
+    } while (0)
+    if (bpc == 1) TDGS_BB(1);
+    else if (bpc == 2) TDGS_BB(2);
+    else if (bpc == 4) TDGS_BB(4);
+    else TDGS_BB(0);
 #undef TDGS_BB
     TDGS_LAUNCHED();
     return TDGS_OK;
