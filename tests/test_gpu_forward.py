@@ -298,3 +298,82 @@ def test_blend_evaluation_counts(gpu):
     e, live, contrib = ev.cpu().tolist()
     covered = int((out.last.cpu().numpy() > 0).sum())
     assert e >= live >= contrib >= covered > 0
+
+
+@pytest.mark.parametrize("tile", [(16, 16), (16, 32), (32, 32), (8, 16), (24, 16), (24, 8), (8, 8), (20, 20)])
+@pytest.mark.parametrize("w,h,depth,last", [(2050, 1702, True, True), (2050, 1702, False, False), (2048, 1600, False, True)])
+def test_render_large_images_bit_exact(gpu, oracle, tile, w, h, depth, last):
+    """Images of many wavefronts (two pixels per lane where the tile is an even number of 8 x 8
+    blocks), ragged and not, with and without the optional outputs."""
+    wl = synthetic.config(0, n=4000)
+    cam = host.look_at_camera(w, h, 60.0, (0.0, 0.0, -4.0))
+    t = host.Tiling.for_camera(cam, *tile)
+    opts = host.RenderOptions.for_camera(cam, 0, background_color=(0.1, 0.2, 0.3))
+    r = oracle.render(wl.gaussians, cam, t, opts)
+    g = gpu.TrainableGaussiansVector.from_host(wl.gaussians, 0)
+    out = gpu.RenderOutputs.for_camera(cam, 0, include_depth=depth, include_last_contributing_indices=last)
+    gpu.render_(out, g, cam, t, opts, gpu.RenderBuffers(len(g), t, 0))
+    np.testing.assert_array_equal(out.rgb.cpu().numpy(), r["rgb"])
+    np.testing.assert_array_equal(out.T.cpu().numpy(), r["T"])
+    if depth:
+        np.testing.assert_array_equal(out.depth.cpu().numpy(), r["depth"])
+    if last:
+        np.testing.assert_array_equal(out.last.cpu().numpy(), r["last"])
+
+
+@pytest.mark.parametrize("k", [1, 3, 5, 127, 130, 257])
+def test_render_list_lengths_at_batch_ends_of_large_images(gpu, oracle, k):
+    """Lists that end 1 to 3 records past a group of four and past batches of 128 records, with two
+    pixels per lane."""
+    cam = host.look_at_camera(2048, 1600, 60.0, (0.0, 0.0, -4.0))
+    t = host.Tiling.for_camera(cam, 16, 16)
+    opts = host.RenderOptions.for_camera(cam, 0, background_color=(0.1, 0.2, 0.3))
+    gh = stacked_faint_gaussians(k)
+    r = oracle.render(gh, cam, t, opts)
+    g = gpu.TrainableGaussiansVector.from_host(gh, 0)
+    out = gpu.RenderOutputs.for_camera(cam, 0)
+    gpu.render_(out, g, cam, t, opts, gpu.RenderBuffers(len(g), t, 0))
+    np.testing.assert_array_equal(out.rgb.cpu().numpy(), r["rgb"])
+    np.testing.assert_array_equal(out.last.cpu().numpy(), r["last"])
+
+
+@pytest.mark.parametrize("min_alpha,max_alpha", [
+    (1 / 255, 0.99), (0.0039, 0.004), (0.05, 0.99), (0.3, 0.99), (0.5, 0.5), (0.75, 0.99), (0.9, 0.99), (0.95, 0.99),
+    (0.5, 0.3), (1.9e-35, 0.99), (1e-36, 0.99), (0.0, 0.99)])
+@pytest.mark.parametrize("w,h", [(256, 256), (2048, 1600)])
+def test_render_alpha_thresholds_bit_exact(gpu, oracle, min_alpha, max_alpha, w, h):
+    """The exponent that stands for min_alpha, over the range of thresholds it is used for and outside it
+    (above 0.9, below exp(-80), above max_alpha, none), where the compares of alpha remain."""
+    wl = synthetic.config(0, n=300)
+    wl.gaussians.means_opacity[:, 3] = np.random.default_rng(1).normal(0.0, 3.0, 300)
+    cam = host.look_at_camera(w, h, 60.0, (0.0, 0.0, -4.0))
+    t = host.Tiling.for_camera(cam, 16, 16)
+    opts = host.RenderOptions.for_camera(cam, 0, min_alpha=min_alpha, max_alpha=max_alpha)
+    r = oracle.render(wl.gaussians, cam, t, opts)
+    g = gpu.TrainableGaussiansVector.from_host(wl.gaussians, 0)
+    out = gpu.RenderOutputs.for_camera(cam, 0)
+    gpu.render_(out, g, cam, t, opts, gpu.RenderBuffers(len(g), t, 0))
+    np.testing.assert_array_equal(out.rgb.cpu().numpy(), r["rgb"])
+    np.testing.assert_array_equal(out.T.cpu().numpy(), r["T"])
+    np.testing.assert_array_equal(out.last.cpu().numpy(), r["last"])
+
+
+@pytest.mark.parametrize("dilation", [0.0, 0.3])
+@pytest.mark.parametrize("w,h", [(256, 256), (2048, 1600)])
+def test_render_extreme_covariances_bit_exact(gpu, oracle, w, h, dilation):
+    """Axes from 1e-6 to 1e6, with and without the dilation: inverse covariances that rounding leaves
+    indefinite, or so narrow for their distance that exponents may pass exp_f's range."""
+    wl = synthetic.config(0, n=300)
+    rng = np.random.default_rng(5)
+    wl.gaussians.scaling[:] = rng.uniform(-14.0, 14.0, wl.gaussians.scaling.shape).astype(np.float32)
+    wl.gaussians.scaling[::3] = rng.uniform(-6.0, 0.0, wl.gaussians.scaling[::3].shape).astype(np.float32)
+    cam = host.look_at_camera(w, h, 60.0, (0.0, 0.0, -4.0))
+    t = host.Tiling.for_camera(cam, 16, 16)
+    opts = host.RenderOptions.for_camera(cam, 0, dilation_x_px=dilation, dilation_y_px=dilation)
+    r = oracle.render(wl.gaussians, cam, t, opts)
+    g = gpu.TrainableGaussiansVector.from_host(wl.gaussians, 0)
+    out = gpu.RenderOutputs.for_camera(cam, 0)
+    gpu.render_(out, g, cam, t, opts, gpu.RenderBuffers(len(g), t, 0))
+    np.testing.assert_array_equal(out.rgb.cpu().numpy(), r["rgb"])
+    np.testing.assert_array_equal(out.T.cpu().numpy(), r["T"])
+    np.testing.assert_array_equal(out.last.cpu().numpy(), r["last"])

@@ -1424,8 +1424,10 @@ struct __align__(16) BlendRec {
 struct BlendArgs {
     int32_t W, H, TW, TH, ntx;
     float bg0, bg1, bg2, min_alpha, max_alpha, min_T;
-    float e_cut;   // exp_f(e) < min_alpha for every exponent e < e_cut
-    int cut_low;   // e_cut < -87: live exponents may leave exp_f's polynomial range
+    float e_cut;     // exp_f(e) < min_alpha for every exponent e < e_cut (with a margin)
+    float e_exact;   // exp_f(e) >= min_alpha exactly for the exponents e >= e_exact
+    int32_t batch;   // records per batch, at most the tile's pixels
+    int checked;     // no such e_exact, or below exp_f's polynomial range: batches take the compiled loop
     int64_t m;
     const int32_t* tiles_end;
     const int32_t* sorted_f;
@@ -1444,27 +1446,31 @@ struct BlendArgs {
     int64_t* mon_host;
 };
 
-// The blending steps of one batch of nb staged records, written out instruction by instruction.
-// Per record it performs exactly the single-precision operations of the C++ loop in
-// k_render_tiles below (same operands, same order: the exponent's five fused multiply-adds,
-// exp_f_core's sequence, min with max_alpha, 1 - alpha, the products and the colour fused
-// multiply-adds; exp_f_core's final product with 2^n is one v_ldexp_f32, which rounds exactly
-// as that product does, subnormal results included), so every result is bit for bit the
-// compiled loop's. What differs is the bookkeeping. Inside the loop exec holds the lanes still
-// blending (act), so every compare yields its mask restricted to them: the live lanes are the
-// compare with e_cut (the exponential is skipped, by a branch on VCC, when none is live), the
-// contributing lanes the compare with min_alpha under exec = live, the stopping lanes the
-// compare with min_T under exec = contributing, and the state update runs under exec =
-// contributing and not stopping; exec is restored on exit. That is 7 scalar and 31 vector
-// instructions per live record (the compiled loop needed about 30 and 39) and 1 scalar
-// instruction per skipped one. The next record (all ten floats) is read from LDS
-// into a second register set while the current one is processed, so no step waits on LDS.
-// Records run in groups of four with one bound check per group (a scalar instruction costs a
-// step about as much as a vector one): after a batch of nb records the LDS array holds three
-// records of padding that no pixel is live for, and one more for the read past the last group.
-// Valid only when every live exponent lies in [-87, 88] (the batch is not `checked`). v39-v63
-// are its scratch registers (the kernel stays within 64 VGPRs, 8 wavefronts per SIMD). Returns
-// the mask of the lanes that did not stop.
+// The blending steps of one batch of staged records, written out instruction by instruction, for one
+// or two pixels per lane (PX). Per record and pixel it performs exactly the single-precision
+// operations of the C++ loop in k_render_tiles below (same operands, same order: the exponent's
+// five fused multiply-adds, exp_f_core's sequence, min with max_alpha, 1 - alpha, the products and
+// the colour fused multiply-adds), so every result is bit for bit the compiled loop's, in cheaper
+// steps:
+//   - the contributing lanes are those with e >= e_exact, one compare for the loop's two (e_cut,
+//     min_alpha): exp_f rises strictly from one float to the next around min_alpha, so
+//     alpha >= min_alpha says the same as e >= e_exact (exact_exponent_cut);
+//   - n = rint(x log2 e) comes from adding and subtracting 1.5 2^23 (the same ties-to-even rounding),
+//     which leaves n in the sum's low mantissa bits; shifted to the exponent field and added to
+//     exp_poly's bits they are the product with 2^n (exact: the exponents are at least -80, so
+//     nothing is subnormal). A compare, a conversion, a v_rndne, an integer or scalar-operand
+//     instruction takes 4 cycles of a SIMD where an add, multiply or FMA takes 2; a v_ldexp with the
+//     conversion it needs takes 8;
+//   - the lanes that would fall below min_T are looked for by one vote; only where there are some (once
+//     per pixel at most) does a detour take them out of act, the mask of the lanes still blending.
+// The next record is read from LDS into a second register set while the current one is processed, so
+// no step waits on LDS. Records run in groups of four with one bound check per group: after a
+// batch the LDS array holds three records of padding that no pixel is live for, and one
+// more for the read past the last group. Valid only for batches that are not `checked`.
+//
+// PX = 2: an LDS read of a record (three reads, 11 cycles of the CU's LDS pipe, shared by its four
+// SIMDs) and the loop's scalar instructions serve two 8 x 8 blocks of the tile; each block is
+// still skipped by itself.
 // the literals of blend_batch's exponential are exp_poly's coefficients
 static_assert(__builtin_bit_cast(uint32_t, kExpC6) == 0x3ab51223u && __builtin_bit_cast(uint32_t, kExpC4) == 0x3d2aac79u &&
                   __builtin_bit_cast(uint32_t, kExpC3) == 0x3e2aaa49u && __builtin_bit_cast(uint32_t, kExpC2) == 0x3efffffeu &&
@@ -1481,257 +1487,236 @@ __device__ __forceinline__ void blend_pad(BlendRec* r) {
     *reinterpret_cast<float2*>(&r->b) = make_float2(z, ninf);
 }
 
-template <bool DEPTH, bool LAST>
-__device__ __forceinline__ uint64_t blend_batch(uint32_t lds_addr, int32_t idx0, int32_t idx_end, float uu,
-                                                float vv, float uv, float cu, float cv, float e_cut,
-                                                float max_alpha, float min_alpha, float min_T, float& T,
-                                                float& C0, float& C1, float& C2, float& D, int32_t& last) {
+// A pixel's accumulators and its position in the tile.
+struct BlendPx {
+    float T, C0, C1, C2, D;
+    int32_t last;
+    float uu, vv, uv, cu, cv;
+};
+
+// Steps through records idx0 .. idx_end - 1 (1-based sorted indices) staged at lds_addr; act[k] is the
+// mask of the lanes whose pixel k is still blending, on entry and on return. v37-v63 are
+// scratch registers (the kernel stays within 64 VGPRs, 8 wavefronts per SIMD).
+template <bool DEPTH, bool LAST, int PX>
+__device__ __forceinline__ void blend_batch(uint32_t lds_addr, int32_t idx0, int32_t idx_end, float e_exact,
+                                            float max_alpha, float min_T, BlendPx (&px)[PX], uint64_t (&act)[PX]) {
     const float c5 = kExpC5;   // exp_poly's coefficient of r^5 (a VGPR operand)
-    uint64_t act, ent, stp;
+    uint64_t ent, lv;
     int32_t idx;
-#define TDGS_BLEND_ASM(DEPTH_FMA, READ_C, LAST_MOV)                                                         \
-    asm volatile(                                                                                           \
-        "s_mov_b64 %[ent], exec\n"                                                                          \
-        "s_and_b64 %[act], exec, exec\n"                                                                    \
-        "s_cbranch_scc0 .Lend_%=\n"                                                                         \
-        "s_mov_b32 %[idx], %[i0]\n"                                                                         \
-        "v_mov_b32 v39, %[addr]\n"                                                                          \
-        "ds_read_b128 v[40:43], v39\n"                                                                      \
-        "ds_read_b128 v[44:47], v39 offset:16\n"                                                            \
-        READ_C("v[48:49]", "v48", "32")                                                                     \
-        ".Lstep_%=:\n"                                                                                      \
-        "s_waitcnt lgkmcnt(0)\n"                                                                            \
-        "ds_read_b128 v[50:53], v39 offset:48\n"                                                            \
-        "ds_read_b128 v[54:57], v39 offset:64\n"                                                            \
-        READ_C("v[58:59]", "v58", "80")                                                                     \
-        "v_fma_f32 v60, v44, %[cv], v45\n"                                                                  \
-        "v_fmac_f32 v60, v43, %[cu]\n"                                                                      \
-        "v_fmac_f32 v60, v42, %[uv]\n"                                                                      \
-        "v_fmac_f32 v60, v41, %[vv]\n"                                                                      \
-        "v_fmac_f32 v60, v40, %[uu]\n"                                                                      \
-        "v_cmp_ngt_f32 vcc, %[cut], v60\n"                                                                  \
-        "s_cbranch_vccz .Ls0_%=\n"                                                                          \
-        "s_mov_b64 exec, vcc\n"                                                                             \
-        "v_mul_f32 v61, 0x3fb8aa3b, v60\n"                                                                  \
-        "v_rndne_f32 v61, v61\n"                                                                            \
-        "v_fmac_f32 v60, 0xbf317200, v61\n"                                                                 \
-        "v_fmac_f32 v60, 0xb5bfbe8e, v61\n"                                                                 \
-        "v_fmamk_f32 v62, v60, 0x3ab51223, %[c5]\n"                                                         \
-        "v_fmaak_f32 v62, v62, v60, 0x3d2aac79\n"                                                           \
-        "v_fmaak_f32 v62, v62, v60, 0x3e2aaa49\n"                                                           \
-        "v_fmaak_f32 v62, v62, v60, 0x3efffffe\n"                                                           \
-        "v_fma_f32 v62, v62, v60, 1.0\n"                                                                    \
-        "v_fma_f32 v62, v62, v60, 1.0\n"                                                                    \
-        "v_cvt_i32_f32 v61, v61\n"                                                                          \
-        "v_ldexp_f32 v62, v62, v61\n"                                                                       \
-        "v_min_f32 v62, %[maxa], v62\n"                                                                     \
-        "v_cmp_ngt_f32 vcc, %[mina], v62\n"                                                                 \
-        "v_sub_f32 v63, 1.0, v62\n"                                                                         \
-        "v_mul_f32 v63, %[T], v63\n"                                                                        \
-        "s_mov_b64 exec, vcc\n"                                                                             \
-        "v_cmp_gt_f32 %[stp], %[minT], v63\n"                                                               \
-        "s_andn2_b64 exec, exec, %[stp]\n"                                                                  \
-        "v_mul_f32 v61, %[T], v62\n"                                                                        \
-        "v_fmac_f32 %[C0], v61, v46\n"                                                                      \
-        "v_fmac_f32 %[C1], v61, v47\n"                                                                      \
-        "v_fmac_f32 %[C2], v61, v48\n"                                                                      \
-        DEPTH_FMA("v49")                                                                                    \
-        "v_mov_b32 %[T], v63\n"                                                                             \
-        LAST_MOV("0")                                                                                       \
-        "s_andn2_b64 %[act], %[act], %[stp]\n"                                                              \
-        "s_mov_b64 exec, %[act]\n"                                                                          \
-        "s_cbranch_scc0 .Lend_%=\n"                                                                         \
-        ".Ls0_%=:\n"                                                                                        \
-        "s_waitcnt lgkmcnt(0)\n"                                                                            \
-        "ds_read_b128 v[40:43], v39 offset:96\n"                                                            \
-        "ds_read_b128 v[44:47], v39 offset:112\n"                                                           \
-        READ_C("v[48:49]", "v48", "128")                                                                    \
-        "v_fma_f32 v60, v54, %[cv], v55\n"                                                                  \
-        "v_fmac_f32 v60, v53, %[cu]\n"                                                                      \
-        "v_fmac_f32 v60, v52, %[uv]\n"                                                                      \
-        "v_fmac_f32 v60, v51, %[vv]\n"                                                                      \
-        "v_fmac_f32 v60, v50, %[uu]\n"                                                                      \
-        "v_cmp_ngt_f32 vcc, %[cut], v60\n"                                                                  \
-        "s_cbranch_vccz .Ls1_%=\n"                                                                          \
-        "s_mov_b64 exec, vcc\n"                                                                             \
-        "v_mul_f32 v61, 0x3fb8aa3b, v60\n"                                                                  \
-        "v_rndne_f32 v61, v61\n"                                                                            \
-        "v_fmac_f32 v60, 0xbf317200, v61\n"                                                                 \
-        "v_fmac_f32 v60, 0xb5bfbe8e, v61\n"                                                                 \
-        "v_fmamk_f32 v62, v60, 0x3ab51223, %[c5]\n"                                                         \
-        "v_fmaak_f32 v62, v62, v60, 0x3d2aac79\n"                                                           \
-        "v_fmaak_f32 v62, v62, v60, 0x3e2aaa49\n"                                                           \
-        "v_fmaak_f32 v62, v62, v60, 0x3efffffe\n"                                                           \
-        "v_fma_f32 v62, v62, v60, 1.0\n"                                                                    \
-        "v_fma_f32 v62, v62, v60, 1.0\n"                                                                    \
-        "v_cvt_i32_f32 v61, v61\n"                                                                          \
-        "v_ldexp_f32 v62, v62, v61\n"                                                                       \
-        "v_min_f32 v62, %[maxa], v62\n"                                                                     \
-        "v_cmp_ngt_f32 vcc, %[mina], v62\n"                                                                 \
-        "v_sub_f32 v63, 1.0, v62\n"                                                                         \
-        "v_mul_f32 v63, %[T], v63\n"                                                                        \
-        "s_mov_b64 exec, vcc\n"                                                                             \
-        "v_cmp_gt_f32 %[stp], %[minT], v63\n"                                                               \
-        "s_andn2_b64 exec, exec, %[stp]\n"                                                                  \
-        "v_mul_f32 v61, %[T], v62\n"                                                                        \
-        "v_fmac_f32 %[C0], v61, v56\n"                                                                      \
-        "v_fmac_f32 %[C1], v61, v57\n"                                                                      \
-        "v_fmac_f32 %[C2], v61, v58\n"                                                                      \
-        DEPTH_FMA("v59")                                                                                    \
-        "v_mov_b32 %[T], v63\n"                                                                             \
-        LAST_MOV("1")                                                                                       \
-        "s_andn2_b64 %[act], %[act], %[stp]\n"                                                              \
-        "s_mov_b64 exec, %[act]\n"                                                                          \
-        "s_cbranch_scc0 .Lend_%=\n"                                                                         \
-        ".Ls1_%=:\n"                                                                                        \
-        "s_waitcnt lgkmcnt(0)\n"                                                                            \
-        "ds_read_b128 v[50:53], v39 offset:144\n"                                                           \
-        "ds_read_b128 v[54:57], v39 offset:160\n"                                                           \
-        READ_C("v[58:59]", "v58", "176")                                                                    \
-        "v_fma_f32 v60, v44, %[cv], v45\n"                                                                  \
-        "v_fmac_f32 v60, v43, %[cu]\n"                                                                      \
-        "v_fmac_f32 v60, v42, %[uv]\n"                                                                      \
-        "v_fmac_f32 v60, v41, %[vv]\n"                                                                      \
-        "v_fmac_f32 v60, v40, %[uu]\n"                                                                      \
-        "v_cmp_ngt_f32 vcc, %[cut], v60\n"                                                                  \
-        "s_cbranch_vccz .Ls2_%=\n"                                                                          \
-        "s_mov_b64 exec, vcc\n"                                                                             \
-        "v_mul_f32 v61, 0x3fb8aa3b, v60\n"                                                                  \
-        "v_rndne_f32 v61, v61\n"                                                                            \
-        "v_fmac_f32 v60, 0xbf317200, v61\n"                                                                 \
-        "v_fmac_f32 v60, 0xb5bfbe8e, v61\n"                                                                 \
-        "v_fmamk_f32 v62, v60, 0x3ab51223, %[c5]\n"                                                         \
-        "v_fmaak_f32 v62, v62, v60, 0x3d2aac79\n"                                                           \
-        "v_fmaak_f32 v62, v62, v60, 0x3e2aaa49\n"                                                           \
-        "v_fmaak_f32 v62, v62, v60, 0x3efffffe\n"                                                           \
-        "v_fma_f32 v62, v62, v60, 1.0\n"                                                                    \
-        "v_fma_f32 v62, v62, v60, 1.0\n"                                                                    \
-        "v_cvt_i32_f32 v61, v61\n"                                                                          \
-        "v_ldexp_f32 v62, v62, v61\n"                                                                       \
-        "v_min_f32 v62, %[maxa], v62\n"                                                                     \
-        "v_cmp_ngt_f32 vcc, %[mina], v62\n"                                                                 \
-        "v_sub_f32 v63, 1.0, v62\n"                                                                         \
-        "v_mul_f32 v63, %[T], v63\n"                                                                        \
-        "s_mov_b64 exec, vcc\n"                                                                             \
-        "v_cmp_gt_f32 %[stp], %[minT], v63\n"                                                               \
-        "s_andn2_b64 exec, exec, %[stp]\n"                                                                  \
-        "v_mul_f32 v61, %[T], v62\n"                                                                        \
-        "v_fmac_f32 %[C0], v61, v46\n"                                                                      \
-        "v_fmac_f32 %[C1], v61, v47\n"                                                                      \
-        "v_fmac_f32 %[C2], v61, v48\n"                                                                      \
-        DEPTH_FMA("v49")                                                                                    \
-        "v_mov_b32 %[T], v63\n"                                                                             \
-        LAST_MOV("2")                                                                                       \
-        "s_andn2_b64 %[act], %[act], %[stp]\n"                                                              \
-        "s_mov_b64 exec, %[act]\n"                                                                          \
-        "s_cbranch_scc0 .Lend_%=\n"                                                                         \
-        ".Ls2_%=:\n"                                                                                        \
-        "s_waitcnt lgkmcnt(0)\n"                                                                            \
-        "ds_read_b128 v[40:43], v39 offset:192\n"                                                           \
-        "ds_read_b128 v[44:47], v39 offset:208\n"                                                           \
-        READ_C("v[48:49]", "v48", "224")                                                                    \
-        "v_fma_f32 v60, v54, %[cv], v55\n"                                                                  \
-        "v_fmac_f32 v60, v53, %[cu]\n"                                                                      \
-        "v_fmac_f32 v60, v52, %[uv]\n"                                                                      \
-        "v_fmac_f32 v60, v51, %[vv]\n"                                                                      \
-        "v_fmac_f32 v60, v50, %[uu]\n"                                                                      \
-        "v_cmp_ngt_f32 vcc, %[cut], v60\n"                                                                  \
-        "s_cbranch_vccz .Ls3_%=\n"                                                                          \
-        "s_mov_b64 exec, vcc\n"                                                                             \
-        "v_mul_f32 v61, 0x3fb8aa3b, v60\n"                                                                  \
-        "v_rndne_f32 v61, v61\n"                                                                            \
-        "v_fmac_f32 v60, 0xbf317200, v61\n"                                                                 \
-        "v_fmac_f32 v60, 0xb5bfbe8e, v61\n"                                                                 \
-        "v_fmamk_f32 v62, v60, 0x3ab51223, %[c5]\n"                                                         \
-        "v_fmaak_f32 v62, v62, v60, 0x3d2aac79\n"                                                           \
-        "v_fmaak_f32 v62, v62, v60, 0x3e2aaa49\n"                                                           \
-        "v_fmaak_f32 v62, v62, v60, 0x3efffffe\n"                                                           \
-        "v_fma_f32 v62, v62, v60, 1.0\n"                                                                    \
-        "v_fma_f32 v62, v62, v60, 1.0\n"                                                                    \
-        "v_cvt_i32_f32 v61, v61\n"                                                                          \
-        "v_ldexp_f32 v62, v62, v61\n"                                                                       \
-        "v_min_f32 v62, %[maxa], v62\n"                                                                     \
-        "v_cmp_ngt_f32 vcc, %[mina], v62\n"                                                                 \
-        "v_sub_f32 v63, 1.0, v62\n"                                                                         \
-        "v_mul_f32 v63, %[T], v63\n"                                                                        \
-        "s_mov_b64 exec, vcc\n"                                                                             \
-        "v_cmp_gt_f32 %[stp], %[minT], v63\n"                                                               \
-        "s_andn2_b64 exec, exec, %[stp]\n"                                                                  \
-        "v_mul_f32 v61, %[T], v62\n"                                                                        \
-        "v_fmac_f32 %[C0], v61, v56\n"                                                                      \
-        "v_fmac_f32 %[C1], v61, v57\n"                                                                      \
-        "v_fmac_f32 %[C2], v61, v58\n"                                                                      \
-        DEPTH_FMA("v59")                                                                                    \
-        "v_mov_b32 %[T], v63\n"                                                                             \
-        LAST_MOV("3")                                                                                       \
-        "s_andn2_b64 %[act], %[act], %[stp]\n"                                                              \
-        "s_mov_b64 exec, %[act]\n"                                                                          \
-        "s_cbranch_scc0 .Lend_%=\n"                                                                         \
-        ".Ls3_%=:\n"                                                                                        \
-        "v_add_u32 v39, 0xc0, v39\n"                                                                        \
-        "s_add_u32 %[idx], %[idx], 4\n"                                                                     \
-        "s_cmp_lt_u32 %[idx], %[iend]\n"                                                                    \
-        "s_cbranch_scc1 .Lstep_%=\n"                                                                        \
-        ".Lend_%=:\n"                                                                                       \
-        "s_waitcnt lgkmcnt(0)\n"                                                                            \
-        "s_mov_b64 exec, %[ent]\n"                                                                          \
-        : [act] "=&s"(act), [ent] "=&s"(ent), [stp] "=&s"(stp),                                       \
-          [idx] "=&s"(idx), [T] "+v"(T), [C0] "+v"(C0), [C1] "+v"(C1), [C2] "+v"(C2), [D] "+v"(D),   \
-          [last] "+v"(last)                                                                         \
-        : [addr] "v"(lds_addr), [i0] "s"(idx0), [iend] "s"(idx_end), [uu] "v"(uu), [vv] "v"(vv),     \
-          [uv] "v"(uv), [cu] "v"(cu), [cv] "v"(cv), [c5] "v"(c5), [cut] "s"(e_cut),                  \
-          [maxa] "s"(max_alpha), [mina] "s"(min_alpha), [minT] "s"(min_T)                           \
-        : "v39", "v40", "v41", "v42", "v43", "v44", "v45", "v46", "v47", "v48", "v49", "v50", "v51",  \
-          "v52", "v53", "v54", "v55", "v56", "v57", "v58", "v59", "v60", "v61", "v62", "v63", "vcc",    \
-          "scc", "memory")
-#define TDGS_DEPTH_ON(R) "v_fmac_f32 %[D], v61, " R "\n"
-#define TDGS_DEPTH_OFF(R) ""
+// exponent of pixel P at the record in registers A0-A3, B0, B1
+#define TDGS_EXPONENT(E, P, A0, A1, A2, A3, B0, B1)  \
+    "v_fma_f32 " E ", " B0 ", %[cv" P "], " B1 "\n"  \
+    "v_fmac_f32 " E ", " A3 ", %[cu" P "]\n"         \
+    "v_fmac_f32 " E ", " A2 ", %[uv" P "]\n"         \
+    "v_fmac_f32 " E ", " A1 ", %[vv" P "]\n"         \
+    "v_fmac_f32 " E ", " A0 ", %[uu" P "]\n"
+// the step of the contributing lanes (exec) of pixel P with exponent E and colour R, G, B
+#define TDGS_LIVE(E, P, ID, K, R, G, B, DEPTH_FMA, LAST_MOV)                                      \
+    "v_mul_f32 v61, 0x3fb8aa3b, " E "\n"                                                              \
+    "v_add_f32 v61, 0x4b400000, v61\n"                                                                \
+    "v_add_f32 v62, 0xcb400000, v61\n"                                                                \
+    "v_fmac_f32 " E ", 0xbf317200, v62\n"                                                             \
+    "v_fmac_f32 " E ", 0xb5bfbe8e, v62\n"                                                             \
+    "v_fmamk_f32 v63, " E ", 0x3ab51223, %[c5]\n"                                                 \
+    "v_fmaak_f32 v63, v63, " E ", 0x3d2aac79\n"                                                   \
+    "v_fmaak_f32 v63, v63, " E ", 0x3e2aaa49\n"                                                   \
+    "v_fmaak_f32 v63, v63, " E ", 0x3efffffe\n"                                                   \
+    "v_fma_f32 v63, v63, " E ", 1.0\n"                                                            \
+    "v_fma_f32 v63, v63, " E ", 1.0\n"                                                            \
+    "v_lshl_add_u32 v63, v61, 23, v63\n"                                                          \
+    "v_min_f32 v63, %[maxa], v63\n"                                                               \
+    "v_sub_f32 v61, 1.0, v63\n"                                                                   \
+    "v_mul_f32 v61, %[T" P "], v61\n"                                                             \
+    "v_cmp_gt_f32 vcc, %[minT], v61\n"                                                            \
+    "s_cbranch_vccnz .Lst" ID P "_%=\n"                                                           \
+    ".Lct" ID P "_%=:\n"                                                                          \
+    "v_mul_f32 v62, %[T" P "], v63\n"                                                             \
+    "v_fmac_f32 %[R" P "], v62, " R "\n"                                                          \
+    "v_fmac_f32 %[G" P "], v62, " G "\n"                                                          \
+    "v_fmac_f32 %[B" P "], v62, " B "\n" DEPTH_FMA "v_mov_b32 %[T" P "], v61\n" LAST_MOV
+// its detour when some of the lanes (vcc) would fall below min_T: they leave act and keep their T
+#define TDGS_STOP1(ID)                               \
+    ".Lst" ID "0_%=:\n"                              \
+    "s_andn2_b64 %[act0], %[act0], vcc\n"            \
+    "s_cbranch_scc0 .Lend_%=\n"                      \
+    "s_andn2_b64 exec, exec, vcc\n"                  \
+    "s_branch .Lct" ID "0_%=\n"
+#define TDGS_STOP2(ID, P)                            \
+    ".Lst" ID P "_%=:\n"                             \
+    "s_andn2_b64 %[act" P "], %[act" P "], vcc\n"    \
+    "s_andn2_b64 exec, exec, vcc\n"                  \
+    "s_or_b64 vcc, %[act0], %[act1]\n"               \
+    "s_cbranch_scc0 .Lend_%=\n"                      \
+    "s_branch .Lct" ID P "_%=\n"
+#define TDGS_READ(READ_C, Q0, Q1, CP, C1, O0, O1, OC)   \
+    "ds_read_b128 " Q0 ", v39 offset:" O0 "\n"          \
+    "ds_read_b128 " Q1 ", v39 offset:" O1 "\n" READ_C(CP, C1, OC)
+// one record: ID = K its number in the group of four, the registers of its set, the next read
+#define TDGS_STEP1(ID, A0, A1, A2, A3, B0, B1, R, G, B, DF, LM, NEXT)                             \
+    "s_waitcnt lgkmcnt(0)\n" NEXT TDGS_EXPONENT("v60", "0", A0, A1, A2, A3, B0, B1)               \
+    "v_cmp_ngt_f32 vcc, %[cut], v60\n"                                                            \
+    "s_cbranch_vccz .Lsk" ID "0_%=\n"                                                             \
+    "s_mov_b64 exec, vcc\n" TDGS_LIVE("v60", "0", ID, ID, R, G, B, DF("0"), LM("0", ID))          \
+    "s_mov_b64 exec, %[act0]\n"                                                                   \
+    ".Lsk" ID "0_%=:\n"
+#define TDGS_STEP2(ID, A0, A1, A2, A3, B0, B1, R, G, B, DF, LM, NEXT)                             \
+    "s_waitcnt lgkmcnt(0)\n" NEXT TDGS_EXPONENT("v60", "0", A0, A1, A2, A3, B0, B1)               \
+    "v_cmp_ngt_f32 vcc, %[cut], v60\n" TDGS_EXPONENT("v38", "1", A0, A1, A2, A3, B0, B1)          \
+    "v_cmp_ngt_f32 %[lv], %[cut], v38\n"                                                          \
+    "s_and_b64 exec, vcc, %[act0]\n"                                                              \
+    "s_cbranch_execz .Lsk" ID "0_%=\n" TDGS_LIVE("v60", "0", ID, ID, R, G, B, DF("0"), LM("0", ID))  \
+    ".Lsk" ID "0_%=:\n"                                                                           \
+    "s_and_b64 exec, %[lv], %[act1]\n"                                                            \
+    "s_cbranch_execz .Lsk" ID "1_%=\n" TDGS_LIVE("v38", "1", ID, ID, R, G, B, DF("1"), LM("1", ID))  \
+    ".Lsk" ID "1_%=:\n"                                                                           \
+    "s_mov_b64 exec, %[ent]\n"
+#define TDGS_SET0 "v40", "v41", "v42", "v43", "v44", "v45", "v46", "v47", "v48"
+#define TDGS_SET1 "v50", "v51", "v52", "v53", "v54", "v55", "v56", "v57", "v58"
+#define TDGS_CALL(F, ...) F(__VA_ARGS__)
+#define TDGS_LOOP(STEP, ENTER, RC, DF0, DF1, LM)                                                              \
+    "s_mov_b64 %[ent], exec\n"                                                                                \
+    "s_mov_b32 %[idx], %[i0]\n"                                                                               \
+    "v_mov_b32 v39, %[addr]\n" TDGS_READ(RC, "v[40:43]", "v[44:47]", "v[48:49]", "v48", "0", "16", "32") ENTER \
+    ".Lstep_%=:\n" TDGS_CALL(STEP, "0", TDGS_SET0, DF0, LM,                                                   \
+                             TDGS_READ(RC, "v[50:53]", "v[54:57]", "v[58:59]", "v58", "48", "64", "80"))      \
+        TDGS_CALL(STEP, "1", TDGS_SET1, DF1, LM,                                                              \
+                  TDGS_READ(RC, "v[40:43]", "v[44:47]", "v[48:49]", "v48", "96", "112", "128"))               \
+            TDGS_CALL(STEP, "2", TDGS_SET0, DF0, LM,                                                          \
+                      TDGS_READ(RC, "v[50:53]", "v[54:57]", "v[58:59]", "v58", "144", "160", "176"))          \
+                TDGS_CALL(STEP, "3", TDGS_SET1, DF1, LM,                                                      \
+                          TDGS_READ(RC, "v[40:43]", "v[44:47]", "v[48:49]", "v48", "192", "208", "224"))      \
+    "v_add_u32 v39, 0xc0, v39\n"                                                                              \
+    "s_add_u32 %[idx], %[idx], 4\n"                                                                           \
+    "s_cmp_lt_u32 %[idx], %[iend]\n"                                                                          \
+    "s_cbranch_scc1 .Lstep_%=\n"                                                                              \
+    "s_branch .Lend_%=\n"
+#define TDGS_TAIL ".Lend_%=:\n" "s_waitcnt lgkmcnt(0)\n" "s_mov_b64 exec, %[ent]\n"
+// (the bound check above runs under whatever exec the last step left; v39 is then advanced for
+// every lane that reads: PX = 1 keeps exec = act0, whose lanes are the only ones that read on)
+#define TDGS_OUT(P, I)                                                                                   \
+    [act##P] "+s"(act[I]), [T##P] "+v"(px[I].T), [R##P] "+v"(px[I].C0), [G##P] "+v"(px[I].C1),            \
+        [B##P] "+v"(px[I].C2)
+// (depth and last index are operands only where they are outputs)
+#define TDGS_OUT_D(P, I) , [D##P] "+v"(px[I].D)
+#define TDGS_OUT_L(P, I) , [L##P] "+v"(px[I].last)
+#define TDGS_OUT_DL(P, I) , [D##P] "+v"(px[I].D), [L##P] "+v"(px[I].last)
+#define TDGS_OUT_NONE(P, I)
+#define TDGS_IN(P, I)                                                                                    \
+    [uu##P] "v"(px[I].uu), [vv##P] "v"(px[I].vv), [uv##P] "v"(px[I].uv), [cu##P] "v"(px[I].cu), [cv##P] "v"(px[I].cv)
+#define TDGS_COMMON_IN                                                                              \
+    [addr] "v"(lds_addr), [i0] "s"(idx0), [iend] "s"(idx_end), [c5] "v"(c5), [cut] "s"(e_exact),     \
+        [maxa] "s"(max_alpha), [minT] "s"(min_T)
+#define TDGS_CLOBBERS                                                                                       \
+    "v38", "v39", "v40", "v41", "v42", "v43", "v44", "v45", "v46", "v47", "v48", "v49", "v50", "v51", "v52", \
+        "v53", "v54", "v55", "v56", "v57", "v58", "v59", "v60", "v61", "v62", "v63", "vcc", "scc", "memory"
+#define TDGS_BLEND1(RC, DF0, DF1, LM, MORE)                                                                           \
+    asm volatile(TDGS_LOOP(TDGS_STEP1, "s_mov_b64 exec, %[act0]\n", RC, DF0, DF1, LM) TDGS_STOP1("0")           \
+                     TDGS_STOP1("1") TDGS_STOP1("2") TDGS_STOP1("3") TDGS_TAIL                                  \
+                 : [ent] "=&s"(ent), [idx] "=&s"(idx), TDGS_OUT(0, 0) MORE(0, 0)                                           \
+                 : TDGS_COMMON_IN, TDGS_IN(0, 0)                                                                \
+                 : TDGS_CLOBBERS)
+#define TDGS_BLEND2(RC, DF0, DF1, LM, MORE)                                                                           \
+    asm volatile(TDGS_LOOP(TDGS_STEP2, "", RC, DF0, DF1, LM) TDGS_STOP2("0", "0") TDGS_STOP2("1", "0")          \
+                     TDGS_STOP2("2", "0") TDGS_STOP2("3", "0") TDGS_STOP2("0", "1") TDGS_STOP2("1", "1")        \
+                         TDGS_STOP2("2", "1") TDGS_STOP2("3", "1") TDGS_TAIL                                    \
+                 : [ent] "=&s"(ent), [idx] "=&s"(idx), [lv] "=&s"(lv), TDGS_OUT(0, 0) MORE(0, 0), TDGS_OUT(1, 1) MORE(1, 1)           \
+                 : TDGS_COMMON_IN, TDGS_IN(0, 0), TDGS_IN(1, 1)                                                 \
+                 : TDGS_CLOBBERS)
+#define TDGS_DEPTH_ON0(P) "v_fmac_f32 %[D" P "], v62, v49\n"
+#define TDGS_DEPTH_ON1(P) "v_fmac_f32 %[D" P "], v62, v59\n"
+#define TDGS_DEPTH_OFF(P) ""
 // the record's last floats: blue and depth (b64), or blue alone (b32) without depth
 #define TDGS_READ_BD(PAIR, ONE, OFF) "ds_read_b64 " PAIR ", v39 offset:" OFF "\n"
 #define TDGS_READ_B(PAIR, ONE, OFF) "ds_read_b32 " ONE ", v39 offset:" OFF "\n"
 // the last contributing index is tracked only when it is an output
-#define TDGS_LAST_ON(K) "v_add_u32_e64 %[last], %[idx], " K "\n"
-#define TDGS_LAST_OFF(K) ""
-    if constexpr (DEPTH && LAST)
-        TDGS_BLEND_ASM(TDGS_DEPTH_ON, TDGS_READ_BD, TDGS_LAST_ON);
-    else if constexpr (DEPTH)
-        TDGS_BLEND_ASM(TDGS_DEPTH_ON, TDGS_READ_BD, TDGS_LAST_OFF);
-    else if constexpr (LAST)
-        TDGS_BLEND_ASM(TDGS_DEPTH_OFF, TDGS_READ_B, TDGS_LAST_ON);
-    else
-        TDGS_BLEND_ASM(TDGS_DEPTH_OFF, TDGS_READ_B, TDGS_LAST_OFF);
-#undef TDGS_BLEND_ASM
-#undef TDGS_DEPTH_ON
+#define TDGS_LAST_ON(P, K) "v_add_u32_e64 %[L" P "], %[idx], " K "\n"
+#define TDGS_LAST_OFF(P, K) ""
+#define TDGS_BLEND(F)                                                                           \
+    do {                                                                                        \
+        if constexpr (DEPTH && LAST) F(TDGS_READ_BD, TDGS_DEPTH_ON0, TDGS_DEPTH_ON1, TDGS_LAST_ON, TDGS_OUT_DL);   \
+        else if constexpr (DEPTH) F(TDGS_READ_BD, TDGS_DEPTH_ON0, TDGS_DEPTH_ON1, TDGS_LAST_OFF, TDGS_OUT_D);     \
+        else if constexpr (LAST) F(TDGS_READ_B, TDGS_DEPTH_OFF, TDGS_DEPTH_OFF, TDGS_LAST_ON, TDGS_OUT_L);        \
+        else F(TDGS_READ_B, TDGS_DEPTH_OFF, TDGS_DEPTH_OFF, TDGS_LAST_OFF, TDGS_OUT_NONE);                           \
+    } while (0)
+    if constexpr (PX == 1) {
+        (void)lv;
+        TDGS_BLEND(TDGS_BLEND1);
+    } else {
+        TDGS_BLEND(TDGS_BLEND2);
+    }
+#undef TDGS_EXPONENT
+#undef TDGS_LIVE
+#undef TDGS_STOP1
+#undef TDGS_STOP2
+#undef TDGS_READ
+#undef TDGS_STEP1
+#undef TDGS_STEP2
+#undef TDGS_SET0
+#undef TDGS_SET1
+#undef TDGS_CALL
+#undef TDGS_LOOP
+#undef TDGS_TAIL
+#undef TDGS_OUT
+#undef TDGS_OUT_D
+#undef TDGS_OUT_L
+#undef TDGS_OUT_DL
+#undef TDGS_OUT_NONE
+#undef TDGS_IN
+#undef TDGS_COMMON_IN
+#undef TDGS_CLOBBERS
+#undef TDGS_BLEND1
+#undef TDGS_BLEND2
+#undef TDGS_DEPTH_ON0
+#undef TDGS_DEPTH_ON1
 #undef TDGS_DEPTH_OFF
 #undef TDGS_READ_BD
 #undef TDGS_READ_B
 #undef TDGS_LAST_ON
 #undef TDGS_LAST_OFF
-    return act;
+#undef TDGS_BLEND
 }
 
-// One workgroup per tile, one thread per pixel (tile_pixel). Each batch of TW*TH sorted
+// One workgroup per tile, one thread per PX pixels (tile_pixel; wavefront w takes pixels 64 PX w + 64 k +
+// lane, k < PX: whole 8 x 8 blocks where PX = 2). Each batch of TW*TH sorted
 // entries is converted to blending parameters once per tile and staged in LDS, where every
-// lane reads the same record (broadcast). A wavefront skips an entry when no pixel it still
-// blends can reach min_alpha (exponent below e_cut), leaves the batch when all its pixels
+// lane reads the same record (broadcast). A wavefront skips an entry for a block when no pixel it
+// still blends can reach min_alpha, leaves the batch when all its pixels
 // are done, and the tile stops loading batches once every pixel is done. The steps of a batch
 // run in blend_batch, except for the counting replay (COUNT) and for batches whose live
-// exponents may leave [-87, 88] (`checked`), which take the loop below with exp_f's range
-// handling.
-template <bool RGB, bool DEPTH, bool COUNT = false, bool LAST = true>
-__global__ __launch_bounds__(1024) void k_render_tiles(BlendArgs a) {
+// exponents may leave [-80, 88] or hold NaN parameters (`checked`), which take the loop below
+// with exp_f's range handling.
+//
+// Two pixels per lane halve the wavefronts, and a wavefront's walk gets longer: it pays only where
+// many rounds of workgroups follow each other (the last one's length no longer counts), and there
+// batches of 128 records, which leave fewer staged in vain behind the pixels' last contributors.
+// us at PX = 1 | PX = 2 with batches of a whole tile | of 128 (in brackets: PX = 1 with the
+// former steps: two compares, v_rndne, conversion and v_ldexp, masks of the stopping lanes): 1M Gaussians 1920x1080 16x16 tiles 132.7 | 143 | 142 (135.0), 16x32 144.6 | 152 | 153
+// (146.8); 1M large ones 1080p 16x32 113.2 | 112.6 | 109.2 (115.0); 3M 2560x1440 16x32 207 | 202.5 |
+// 197.6 (208.6); 1M 3840x2160 16x32 441 | 426 | 413 (444.8), 16x16 410 | 412 | 404 (415); 3M large
+// ones 3840x2160 16x32 386 | 363 | 347 (394.5). The line lies between 1080p (16200 wavefronts at
+// PX = 2) and 1440p (28800).
+constexpr int64_t kBlendWaves2 = 24576;
+constexpr int kBlendBatch2 = 128;
+template <bool RGB, bool DEPTH, bool COUNT = false, bool LAST = true, int PX = 1>
+__global__ __launch_bounds__(1024 / PX) __attribute__((amdgpu_waves_per_eu(PX == 1 ? 8 : 6))) void k_render_tiles(BlendArgs a) {
     extern __shared__ BlendRec s_rec[];
     const int NT = a.TW * a.TH;
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, NTH = NT / PX, NB = a.batch;
     const int tx = blockIdx.x + 1, ty = blockIdx.y + 1;
     const int tile = tx + (ty - 1) * a.ntx;
-    int u_in, v_in;
-    tile_pixel(t, a.TW, a.TH, &u_in, &v_in);
-    const int U = u_in + (tx - 1) * a.TW, V = v_in + (ty - 1) * a.TH;
-    const bool on = U <= a.W && V <= a.H;
-    const float cu = (float)u_in - 0.5f, cv = (float)v_in - 0.5f;
-    const float uu = cu * cu, uv = cu * cv, vv = cv * cv;
     const float u0 = (float)((tx - 1) * a.TW), v0 = (float)((ty - 1) * a.TH);
+    const float side = (float)(a.TW > a.TH ? a.TW : a.TH);
+    BlendPx px[PX];
+    bool on[PX], done[PX];
+#pragma unroll
+    for (int k = 0; k < PX; ++k) {
+        int u_in, v_in;
+        tile_pixel(PX == 1 ? t : (t / kWave) * (PX * kWave) + k * kWave + (t % kWave), a.TW, a.TH, &u_in, &v_in);
+        const float cu = (float)u_in - 0.5f, cv = (float)v_in - 0.5f;
+        px[k] = {1.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0, cu * cu, cv * cv, cu * cv, cu, cv};
+        on[k] = u_in + (tx - 1) * a.TW <= a.W && v_in + (ty - 1) * a.TH <= a.H;
+        done[k] = !on[k];
+    }
     int64_t m = a.m;
     bool nothing = false;   // render_void!'s outputs (a device-count render with no keys)
     if (!COUNT && a.dcount) {
@@ -1759,49 +1744,70 @@ __global__ __launch_bounds__(1024) void k_render_tiles(BlendArgs a) {
     if (beg < 0) beg = 0;
     if (beg > end) beg = end;
 
-    float T = 1.0f, C0 = 0.0f, C1 = 0.0f, C2 = 0.0f, D = 0.0f;
-    int32_t last = 0;
-    bool done = !on;
     unsigned long long evals = 0, live_n = 0, contrib_n = 0;
     // blend_batch runs records in groups of four: up to three records after a batch are padding
     // that no pixel is live for (exponent -inf), written where a batch ends
-    for (int k = t; k < 3; k += NT) blend_pad(s_rec + NT + k);   // (tiles of fewer than 3 pixels too)
-    for (int64_t base = beg; base < end; base += NT) {
-        if (__syncthreads_count(done ? 0 : 1) == 0) break;
-        const int64_t s = base + t;
-        bool big = false;   // opacity above 1e38: exponents may pass 88
-        if (s >= end && s < end + 3) blend_pad(s_rec + t);
-        if (s < end) {
-            const int64_t f = (int64_t)a.sorted_f[s] - 1;
-            const float* r = a.f2d + 9 * f;
-            float p[6];
-            blend_params(r[0], r[1], r[2], r[3], r[4], r[5], u0, v0, p);
-            BlendRec rec;
-            rec.a = make_float4(p[0], p[1], p[2], p[3]);
-            rec.b = make_float4(p[4], p[5], RGB ? r[6] : 0.0f, RGB ? r[7] : 0.0f);
-            rec.c = make_float4(RGB ? r[8] : 0.0f, DEPTH ? a.depths[f] : 0.0f, 0.0f, 0.0f);
-            s_rec[t] = rec;
-            big = !(r[2] <= 1e38f);
-        }
-        // A live exponent lies in [e_cut, log a]; unless e_cut < -87 or an opacity in the
-        // batch is huge (or NaN), that is inside [-87, 88], where exp_f is its polynomial core.
-        const bool checked = __syncthreads_or(big) || a.cut_low;
-        const int nb = (int)((end - base) < NT ? (end - base) : NT);
-        if (!COUNT && !checked) {
-            if (!done) {
-                const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) BlendRec*)s_rec;
-                const uint64_t act = blend_batch<DEPTH, LAST>(lds, (int32_t)(base + 1), (int32_t)(base + nb + 1), uu,
-                                                        vv, uv, cu, cv, a.e_cut, a.max_alpha, a.min_alpha,
-                                                        a.min_T, T, C0, C1, C2, D, last);
-                done = ((act >> __lane_id()) & 1ull) == 0;
+    for (int k = t; k < 3; k += NTH) blend_pad(s_rec + NB + k);   // (tiles of fewer than 3 pixels too)
+    for (int64_t base = beg; base < end; base += NB) {
+        bool all_done = done[0];
+        if (PX == 2) all_done = all_done && done[PX - 1];
+        if (__syncthreads_count(all_done ? 0 : 1) == 0) break;
+        // A record whose exponents might pass 88, or be NaN: parameters that are no numbers, an opacity
+        // above 1e9 (log a > 20), an inverse covariance that is not (within 1e-6) definite, or one so
+        // narrow for its distance that rounding or that 1e-6 could lift the exponent by 65.
+        bool odd = false;
+#pragma unroll
+        for (int k = 0; k < PX; ++k) {
+            const int i = t + k * NTH;
+            const int64_t s = i < NB ? base + i : end + 3;
+            if (s >= end && s < end + 3) blend_pad(s_rec + i);
+            if (s < end) {
+                const int64_t f = (int64_t)a.sorted_f[s] - 1;
+                const float* r = a.f2d + 9 * f;
+                float p[6];
+                blend_params(r[0], r[1], r[2], r[3], r[4], r[5], u0, v0, p);
+                BlendRec rec;
+                rec.a = make_float4(p[0], p[1], p[2], p[3]);
+                rec.b = make_float4(p[4], p[5], RGB ? r[6] : 0.0f, RGB ? r[7] : 0.0f);
+                rec.c = make_float4(RGB ? r[8] : 0.0f, DEPTH ? a.depths[f] : 0.0f, 0.0f, 0.0f);
+                s_rec[i] = rec;
+                const float reach = fabsf(r[0] - u0) + fabsf(r[1] - v0) + side;   // (NaN with either)
+                const bool plain = r[2] >= 0.0f && r[2] <= 1e9f && p[0] <= 0.0f && p[1] <= 0.0f &&
+                                   p[2] * p[2] <= 4.000004f * p[0] * p[1] &&
+                                   (fabsf(p[0]) + fabsf(p[1]) + fabsf(p[2])) * reach * reach <= 1e8f;
+                odd = odd || !plain;
             }
-        } else if (!done) {
+        }
+        // A live exponent lies in [e_exact, log a + 65]; unless e_exact < -80 or a record of the
+        // batch is odd, that is inside [-87, 88], where exp_f is its polynomial core.
+        const bool checked = __syncthreads_or(odd) || a.checked;
+        const int nb = (int)((end - base) < NB ? (end - base) : NB);
+        if (!COUNT && !checked) {
+            uint64_t act[PX], any = 0;
+#pragma unroll
+            for (int k = 0; k < PX; ++k) {
+                act[k] = __builtin_amdgcn_ballot_w64(!done[k]);
+                any |= act[k];
+            }
+            if (any != 0) {
+                const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) BlendRec*)s_rec;
+                blend_batch<DEPTH, LAST, PX>(lds, (int32_t)(base + 1), (int32_t)(base + nb + 1), a.e_exact,
+                                             a.max_alpha, a.min_T, px, act);
+#pragma unroll
+                for (int k = 0; k < PX; ++k) done[k] = ((act[k] >> __lane_id()) & 1ull) == 0;
+            }
+            continue;
+        }
+#pragma unroll
+        for (int k = 0; k < PX; ++k) {
+            BlendPx& q = px[k];
+            if (done[k]) continue;
             for (int j = 0; j < nb; ++j) {
-                if (COUNT && !done) ++evals;
+                if (COUNT && !done[k]) ++evals;
                 const float4 ra = s_rec[j].a;
                 const float4 rb = s_rec[j].b;
-                const float e = fmaf(ra.x, uu, fmaf(ra.y, vv, fmaf(ra.z, uv, fmaf(ra.w, cu, fmaf(rb.x, cv, rb.y)))));
-                const bool live = !done && !(e < a.e_cut);
+                const float e = fmaf(ra.x, q.uu, fmaf(ra.y, q.vv, fmaf(ra.z, q.uv, fmaf(ra.w, q.cu, fmaf(rb.x, q.cv, rb.y)))));
+                const bool live = !done[k] && !(e < a.e_cut);
                 if (!wave_any(live)) continue;
                 // exp_f(e) for the live lanes: the polynomial core unless a live lane is outside
                 // [-87, 88] or NaN (the other lanes' values are not used)
@@ -1815,25 +1821,25 @@ __global__ __launch_bounds__(1024) void k_render_tiles(BlendArgs a) {
                     live_n += live ? 1 : 0;
                     contrib_n += contrib ? 1 : 0;
                 }
-                const float Tn = T * (1.0f - alpha);
+                const float Tn = q.T * (1.0f - alpha);
                 const bool stop = contrib && Tn < a.min_T;
                 if (contrib && !stop) {
-                    const float w = T * alpha;
+                    const float w = q.T * alpha;
                     if (RGB || DEPTH) {
                         const float4 rc = s_rec[j].c;
                         if (RGB) {
-                            C0 = fmaf(w, rb.z, C0);
-                            C1 = fmaf(w, rb.w, C1);
-                            C2 = fmaf(w, rc.x, C2);
+                            q.C0 = fmaf(w, rb.z, q.C0);
+                            q.C1 = fmaf(w, rb.w, q.C1);
+                            q.C2 = fmaf(w, rc.x, q.C2);
                         }
-                        if (DEPTH) D = fmaf(w, rc.y, D);
+                        if (DEPTH) q.D = fmaf(w, rc.y, q.D);
                     }
-                    T = Tn;
-                    last = (int32_t)(base + j + 1);
+                    q.T = Tn;
+                    q.last = (int32_t)(base + j + 1);
                 }
                 if (wave_any(stop)) {
-                    done = done || stop;
-                    if (!wave_any(!done)) break;
+                    done[k] = done[k] || stop;
+                    if (!wave_any(!done[k])) break;
                 }
             }
         }
@@ -1851,16 +1857,22 @@ __global__ __launch_bounds__(1024) void k_render_tiles(BlendArgs a) {
         }
         return;
     }
-    if (!on) return;
-    const int64_t px = (int64_t)(V - 1) + (int64_t)a.H * (U - 1);
-    if (RGB && a.rgb) {
-        a.rgb[3 * px] = fmaf(T, a.bg0, C0);
-        a.rgb[3 * px + 1] = fmaf(T, a.bg1, C1);
-        a.rgb[3 * px + 2] = fmaf(T, a.bg2, C2);
+#pragma unroll
+    for (int k = 0; k < PX; ++k) {
+        if (!on[k]) continue;
+        const BlendPx& q = px[k];
+        int u_in, v_in;
+        tile_pixel(PX == 1 ? t : (t / kWave) * (PX * kWave) + k * kWave + (t % kWave), a.TW, a.TH, &u_in, &v_in);
+        const int64_t at = (int64_t)(v_in + (ty - 1) * a.TH - 1) + (int64_t)a.H * (u_in + (tx - 1) * a.TW - 1);
+        if (RGB && a.rgb) {
+            a.rgb[3 * at] = fmaf(q.T, a.bg0, q.C0);
+            a.rgb[3 * at + 1] = fmaf(q.T, a.bg1, q.C1);
+            a.rgb[3 * at + 2] = fmaf(q.T, a.bg2, q.C2);
+        }
+        if (a.T) a.T[at] = q.T;
+        if (DEPTH && a.depth) a.depth[at] = nothing ? kInf : q.D;
+        if (a.last) a.last[at] = q.last;
     }
-    if (a.T) a.T[px] = T;
-    if (DEPTH && a.depth) a.depth[px] = nothing ? kInf : D;
-    if (a.last) a.last[px] = last;
 }
 
 // render_void! (forward_structs.jl:743-757).
@@ -1900,7 +1912,7 @@ static int launch_render_tiles(hipStream_t s, const tdgs_camera* cam, const tdgs
     a.bg0 = o->background[0]; a.bg1 = o->background[1]; a.bg2 = o->background[2];
     a.min_alpha = o->min_alpha; a.max_alpha = o->max_alpha; a.min_T = o->min_transmittance;
     a.e_cut = exponent_cut(o->min_alpha);
-    a.cut_low = !(a.e_cut >= -87.0f);
+    a.checked = !exact_exponent_cut(o->min_alpha, o->max_alpha, &a.e_exact);
     a.m = m; a.tiles_end = tiles_end; a.sorted_f = sorted_f; a.f2d = f2d; a.depths = depths;
     a.rgb = out->rgb; a.T = out->T; a.depth = out->depth; a.last = out->last;
     a.evaluations = evaluations;
@@ -1911,7 +1923,13 @@ static int launch_render_tiles(hipStream_t s, const tdgs_camera* cam, const tdgs
     const int nt = t->tile_width * t->tile_height;
     const dim3 grid(t->nb_tiles_x, t->nb_tiles_y);
     // + the padding after a batch and the record blend_batch reads past its last group of four
-    const size_t lds = (size_t)(nt + 4) * sizeof(BlendRec);
+    // Two pixels per lane where that leaves at least three rounds of the chip's 8192 wavefronts: see
+    // k_render_tiles.
+    const int64_t waves2 = (int64_t)t->nb_tiles_x * t->nb_tiles_y * (nt / (2 * kWave));
+    const bool two = t->tile_width % 8 == 0 && t->tile_height % 8 == 0 && nt % (2 * kWave) == 0 &&
+                     waves2 >= kBlendWaves2 && !evaluations;
+    a.batch = two ? kBlendBatch2 : nt;
+    const size_t lds = (size_t)(a.batch + 4) * sizeof(BlendRec);
     if (evaluations) {
         k_render_tiles<false, false, true><<<grid, nt, lds, s>>>(a);
         TDGS_LAUNCHED();
@@ -1919,19 +1937,25 @@ static int launch_render_tiles(hipStream_t s, const tdgs_camera* cam, const tdgs
     }
     const bool rgb = out->rgb != nullptr, dep = out->depth != nullptr;
     const bool last = out->last != nullptr;
+#define TDGS_RT(RGB_, DEP_, LAST_)                                                             \
+    do {                                                                                       \
+        if (two) k_render_tiles<RGB_, DEP_, false, LAST_, 2><<<grid, nt / 2, lds, s>>>(a);     \
+        else k_render_tiles<RGB_, DEP_, false, LAST_, 1><<<grid, nt, lds, s>>>(a);             \
+    } while (0)
     if (rgb && dep) {
-        if (last) k_render_tiles<true, true, false, true><<<grid, nt, lds, s>>>(a);
-        else k_render_tiles<true, true, false, false><<<grid, nt, lds, s>>>(a);
+        if (last) TDGS_RT(true, true, true);
+        else TDGS_RT(true, true, false);
     } else if (rgb) {
-        if (last) k_render_tiles<true, false, false, true><<<grid, nt, lds, s>>>(a);
-        else k_render_tiles<true, false, false, false><<<grid, nt, lds, s>>>(a);
+        if (last) TDGS_RT(true, false, true);
+        else TDGS_RT(true, false, false);
     } else if (dep) {
-        if (last) k_render_tiles<false, true, false, true><<<grid, nt, lds, s>>>(a);
-        else k_render_tiles<false, true, false, false><<<grid, nt, lds, s>>>(a);
+        if (last) TDGS_RT(false, true, true);
+        else TDGS_RT(false, true, false);
     } else {
-        if (last) k_render_tiles<false, false, false, true><<<grid, nt, lds, s>>>(a);
-        else k_render_tiles<false, false, false, false><<<grid, nt, lds, s>>>(a);
+        if (last) TDGS_RT(false, false, true);
+        else TDGS_RT(false, false, false);
     }
+#undef TDGS_RT
     TDGS_LAUNCHED();
     return TDGS_OK;
 }

@@ -63,6 +63,30 @@ inline float exponent_cut(float min_alpha) {
     return std::nextafter((float)(std::log((double)min_alpha) - 1e-3), -__builtin_inff());
 }
 
+// The exponent from which alpha = exp_f(e) reaches min_alpha: exp_f(e) >= min_alpha exactly for e >= *cut.
+// Around a min_alpha of at most 0.9 neighbouring exponents are at least 7e-9 apart and exp_f is within
+// 0.91 ulp (1.1e-7) of a strictly rising function, so the switch is looked for within 32 floats of
+// log(min_alpha) and has to be a clean one there (further away the order is certain). False when there
+// is none, when max_alpha stays below min_alpha, or when *cut < -80 (results of exp_f near its
+// flush to zero).
+inline bool exact_exponent_cut(float min_alpha, float max_alpha, float* cut) {
+    *cut = 0.0f;
+    if (!(min_alpha > 0.0f) || !(min_alpha <= 0.9f) || !(max_alpha >= min_alpha)) return false;
+    constexpr int kSpan = 32;
+    float e = (float)std::log((double)min_alpha);
+    if (!(e >= -80.0f)) return false;
+    for (int k = 0; k < kSpan; ++k) e = std::nextafter(e, -kInf);
+    bool reached = false;
+    for (int k = 0; k < 2 * kSpan; ++k, e = std::nextafter(e, kInf)) {
+        const bool r = exp_f(e) >= min_alpha;
+        if (r && !reached) *cut = e;
+        if (!r && reached) return false;
+        reached = r;
+        if (r && k == 0) return false;
+    }
+    return reached;
+}
+
 // Pixel of thread t inside a TW x TH tile (1-based). With both sides multiples of 8 each
 // wavefront covers an 8x8 block (blocks column-major, lanes column-major inside), which
 // keeps a Gaussian's footprint inside as few wavefronts as possible; otherwise wavefront
