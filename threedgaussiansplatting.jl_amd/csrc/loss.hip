@@ -50,6 +50,21 @@ struct SsimWindow {
     float w[2 * kSsimR + 1];
 };
 
+// The window in vector registers (it is symmetric: six of them). As kernel arguments the weights are
+// scalar registers, and a VALU instruction with a scalar operand takes twice the issue cycles (4.9
+// against 2.7, measured); the empty asm keeps the compiler from going back to them.
+struct SsimWeights {
+    float w[kSsimR + 1];
+    __device__ __forceinline__ explicit SsimWeights(const SsimWindow& win) {
+#pragma unroll
+        for (int k = 0; k <= kSsimR; ++k) {
+            w[k] = win.w[k];
+            asm volatile("" : "+v"(w[k]));
+        }
+    }
+    __device__ __forceinline__ float operator[](int d) const { return w[d <= kSsimR ? d : 2 * kSsimR - d]; }
+};
+
 // The backward pass reads the derivative maps through a buffer descriptor: one uniform base,
 // 32-bit offsets (map q at the scalar offset 4 q P), and a range check that returns 0 for the
 // taps outside the image (offset kNoTap, past the buffer: tdgs_loss_grad takes images of fewer
@@ -84,6 +99,7 @@ __global__ __launch_bounds__(256) void k_ssim_forward(const float* __restrict__ 
     int tv, tu;
     ssim_tile((H + kSsimT - 1) / kSsimT, gridDim.x, &tv, &tu);
     const int v0 = tv * kSsimT - kSsimR, u0 = tu * kSsimT - kSsimR;
+    const SsimWeights ww(win);
     // the tile's inputs: pixel k = t + 256 i (i < 3) of the 26 x 26 tile, all loads issued
     // before the first LDS store (pixel indices are 32-bit: tdgs_loss_grad takes images of fewer
     // than 2^31 / 9 pixels)
@@ -139,11 +155,11 @@ __global__ __launch_bounds__(256) void k_ssim_forward(const float* __restrict__ 
         for (int o = 0; o < 6; ++o) {
             if (o >= no) break;
             // (the first tap as a product: no zeroed accumulators)
-            const float w0 = win.w[0], a0 = a[o], b0 = b[o];
+            const float w0 = ww[0], a0 = a[o], b0 = b[o];
             float m0 = w0 * a0, m1 = w0 * b0, m2 = w0 * (a0 * a0), m3 = w0 * (b0 * b0), m4 = w0 * (a0 * b0);
 #pragma unroll
             for (int d = 1; d < 2 * kSsimR + 1; ++d) {
-                const float wd = win.w[d], av = a[o + d], bv = b[o + d];
+                const float wd = ww[d], av = a[o + d], bv = b[o + d];
                 m0 = fmaf(wd, av, m0);
                 m1 = fmaf(wd, bv, m1);
                 m2 = fmaf(wd, av * av, m2);
@@ -173,9 +189,9 @@ __global__ __launch_bounds__(256) void k_ssim_forward(const float* __restrict__ 
     if (p2) {
 #pragma unroll
         for (int ou = 0; ou < kSsimT; ++ou) {
-            float m = win.w[0] * f[ou];
+            float m = ww[0] * f[ou];
 #pragma unroll
-            for (int d = 1; d < 2 * kSsimR + 1; ++d) m = fmaf(win.w[d], f[ou + d], m);
+            for (int d = 1; d < 2 * kSsimR + 1; ++d) m = fmaf(ww[d], f[ou + d], m);
             s_out[(ou * kSsimT + p2_ov) * kOutPitch + p2_q] = m;
         }
     }
@@ -272,6 +288,7 @@ __global__ __launch_bounds__(256) void k_ssim_backward(const float* __restrict__
     int tv, tu;
     ssim_tile((H + kSsimT - 1) / kSsimT, gridDim.x, &tv, &tu);
     const int v0 = tv * kSsimT - kSsimR, u0 = tu * kSsimT - kSsimR;
+    const SsimWeights ww(win);
     if (blockIdx.x == 0) ssim_add_partials(partials, nblk, sums);
     // this thread's output pixel and its inputs (read now, used at the end)
     const int ov = t % kSsimT, ou = t / kSsimT;
@@ -325,9 +342,9 @@ __global__ __launch_bounds__(256) void k_ssim_backward(const float* __restrict__
         const int iu = t / kQB, q = t % kQB;
 #pragma unroll
         for (int ov = 0; ov < kSsimT; ++ov) {
-            float m = win.w[0] * a[ov];
+            float m = ww[0] * a[ov];
 #pragma unroll
-            for (int d = 1; d < 2 * kSsimR + 1; ++d) m = fmaf(win.w[d], a[ov + d], m);
+            for (int d = 1; d < 2 * kSsimR + 1; ++d) m = fmaf(ww[d], a[ov + d], m);
             s_v[(q * kSsimT + ov) * kRow + iu] = m;
         }
     }
@@ -346,9 +363,9 @@ __global__ __launch_bounds__(256) void k_ssim_backward(const float* __restrict__
         const int ov = t % kSsimT, q = t / kSsimT;
 #pragma unroll
         for (int ou = 0; ou < kSsimT; ++ou) {
-            float m = win.w[0] * b[ou];
+            float m = ww[0] * b[ou];
 #pragma unroll
-            for (int d = 1; d < 2 * kSsimR + 1; ++d) m = fmaf(win.w[d], b[ou + d], m);
+            for (int d = 1; d < 2 * kSsimR + 1; ++d) m = fmaf(ww[d], b[ou + d], m);
             s_out[(ou * kSsimT + ov) * kOutPitch + q] = m;
         }
     }
