@@ -251,3 +251,34 @@ def test_kept_but_nothing_on_screen(gpu, oracle, device_counts):
     np.testing.assert_array_equal(out.rgb.cpu().numpy(), r["rgb"])
     np.testing.assert_array_equal(out.T.cpu().numpy(), r["T"])
     assert np.all(out.T.cpu().numpy() == 1) and np.all(out.last.cpu().numpy() == 0)
+
+
+@pytest.mark.parametrize("n", [1, 511, 513, 1025, 4097])
+@pytest.mark.parametrize("w,h,tile", [(256, 200, (16, 16)), (1285, 700, (16, 16)), (1920, 1080, (8, 8)), (1020, 1020, (4, 4))])
+def test_small_scene_lists_match_oracle(gpu, oracle, n, w, h, tile):
+    """Tile lists made straight from the depth-ordered Gaussians (few blocks x Gaussians), in blocks of
+    8 x 8, 16 x 8 and 16 x 16 tiles, at the ends of the chunks a workgroup takes, with the counts on the
+    device and on the host; with key arrays too small for their count table (the coarse lists then),
+    and with too few keys."""
+    g_host = synthetic.config(0, n=n).gaussians
+    cam = host.look_at_camera(w, h, 60.0, (0.0, 0.0, -4.0))
+    t = host.Tiling.for_camera(cam, *tile)
+    opts = host.RenderOptions.for_camera(cam, 0, background_color=(0.1, 0.2, 0.3))
+    r = oracle.render(g_host, cam, t, opts)
+    g = gpu.TrainableGaussiansVector.from_host(g_host, 0)
+    for key_capacity in (max(r["nb_keys"], 1), 40 * n + 40_000 + r["nb_keys"]):
+        out, buf = _device_render(gpu, g, cam, t, opts, key_capacity=key_capacity)
+        nbf, m, nb, status = buf.frame_counts()
+        assert (nbf, m, status) == (r["nb_fgaussians"], r["nb_keys"], abi.TDGS_FRAME_OK)
+        _assert_forward_equal(r, out, buf)
+        out = gpu.RenderOutputs.for_camera(cam, 0, include_depth=True)
+        buf = gpu.RenderBuffers(len(g), t, 0, key_capacity, keep_flags=True)
+        gpu.render_(out, g, cam, t, opts, buf)
+        torch.cuda.synchronize()
+        _assert_forward_equal(r, out, buf)
+    if r["nb_keys"] > 1:
+        out, buf = _device_render(gpu, g, cam, t, opts, key_capacity=r["nb_keys"] - 1)
+        nbf, m, nb, status = buf.frame_counts()
+        assert (nbf, m, status) == (r["nb_fgaussians"], r["nb_keys"], abi.TDGS_FRAME_KEY_CAPACITY)
+        assert float(out.T.min()) == 1.0 and int(out.last.max()) == 0
+    gpu.ctx_check(0)

@@ -33,6 +33,7 @@
 // without sorting the M keys; the 64-bit keys are assembled only on request
 // (tdgs_render_sorted_keys).
 #include <mutex>
+#include <type_traits>
 
 #include "dsort.hpp"
 #include "internal.hpp"
@@ -985,12 +986,17 @@ struct BinArgs {
     const int64_t* dmc;        // entries used (device counts), or null
     const int32_t* ranges;     // tile rectangles [x0, y0, x1, y1] (1-based, inclusive) by fgidx
     const uint32_t* cmask;     // or null: each entry's tiles of its block (EmitGrid::block_mask)
-    int32_t* table;            // COUNT writes the Gaussians of each segment covering each tile
+    void* table;               // COUNT writes the Gaussians of each segment covering each tile
     int32_t* tile_totals;      // COUNT adds them up per tile (zeroed beforehand)
     const int32_t* tiles_end;  // WRITE: inclusive ends of the tiles' lists
     int32_t* out;              // WRITE: sdfgidx_to_fgidx
     int32_t cap;               // WRITE: entries of out
     uint32_t* err;
+    // DIRECT: every block's candidates are all non-empty Gaussians in depth order
+    const int4* srect;         // their rectangles
+    const int32_t* sorted_f;   // and fgidx
+    int64_t nb;                // how many (launch bound)
+    const int64_t* dnb;        // how many (device counts), or null
 };
 
 // Workgroup: 4 threads per tile of a block of 2^SX x 2^sy tiles; wavefront w takes the
@@ -1002,7 +1008,10 @@ struct BinArgs {
 // earlier segments' hits + the hits before it.
 // (Staging the writes in LDS rings and storing 64 entries at a time measured no faster.)
 // LDS (dynamic): the chunk's candidates, 2 bin_per(SX) words per thread.
-template <int SX, bool WRITE>
+// DIRECT (small scenes): no coarse list. Chunk k = b cpb + c tests the c-th run of nt of all
+// Gaussians against block b (cpb = ceil(N_b / nt)), the masks made from the contiguous depth-ordered
+// rectangles; its counts are table[k tpb + local tile]. See direct_lists.
+template <int SX, bool WRITE, bool DIRECT>
 __global__ __launch_bounds__(1024) void k_bin_tiles(BinArgs a) {
     extern __shared__ uint32_t s_dyn[];
     __shared__ int32_t s_cend[1024];   // the blocks' ends, when there are at most 1024 blocks
@@ -1013,14 +1022,20 @@ __global__ __launch_bounds__(1024) void k_bin_tiles(BinArgs a) {
     constexpr int BW = 1 << SX;
     const int BH = 1 << a.sy;
     const int tpb = BW * BH;
+    // (DIRECT's table has a row per block and chunk: 16-bit counts, a chunk's entries are at most 4096)
+    using BinCount = std::conditional_t<DIRECT, uint16_t, int32_t>;
+    BinCount* const table = static_cast<BinCount*>(a.table);
     const int t = threadIdx.x, lane = __lane_id(), w = t / kWave;
     const int nt = (int)blockDim.x * PER;   // entries per chunk
-    int64_t mc = a.mc;
-    if (a.dmc && *a.dmc < mc) mc = *a.dmc;
-    const int64_t nchunks = (mc + nt - 1) / nt;
+    int64_t mc = DIRECT ? a.nb : a.mc;
+    if (DIRECT && a.dnb && *a.dnb < mc) mc = *a.dnb;
+    if (a.dmc && (DIRECT ? *a.dmc == 0 : *a.dmc < mc)) mc = DIRECT ? 0 : *a.dmc;
+    const int64_t cpb = (mc + nt - 1) / nt;   // DIRECT: chunks per block
+    const int64_t nchunks = DIRECT ? cpb * a.nblocks : cpb;
     if ((int64_t)blockIdx.x >= nchunks) return;
     const bool lds_ends = a.nblocks <= 1024;
-    if (a.totals) {
+    if (DIRECT) {
+    } else if (a.totals) {
         // one radix pass sorted the 8-bit block ids (at most 255 blocks, at least 256
         // threads): the ends are the inclusive prefix sums of the digit totals 1..255
         const int lane = __lane_id();
@@ -1046,7 +1061,11 @@ __global__ __launch_bounds__(1024) void k_bin_tiles(BinArgs a) {
     const int li = 16 * w + lane;     // lanes < 16: the tile this lane reports (local index)
     const int ly0 = (16 * w) >> SX;   // the wavefront's first local row
     for (int64_t k = blockIdx.x; k < nchunks; k += gridDim.x) {
-        const int64_t lo = k * nt, hi = lo + nt < mc ? lo + nt : mc;
+        const int64_t lo = (DIRECT ? k % cpb : k) * nt, hi = lo + nt < mc ? lo + nt : mc;
+        int b0 = 0, b1 = 0;
+        if constexpr (DIRECT) {
+            b0 = b1 = (int)(k / cpb);
+        } else {
         // the blocks holding entries lo and hi - 1 (the ends never decrease): counts of the
         // blocks ending at or before lo, and before hi
         if (t == 0) s_b[0] = s_b[1] = 0;
@@ -1066,17 +1085,19 @@ __global__ __launch_bounds__(1024) void k_bin_tiles(BinArgs a) {
             atomicAdd(&s_b[1], c1);
         }
         __syncthreads();
-        const int b0 = s_b[0], b1 = s_b[1];
+        b0 = s_b[0];
+        b1 = s_b[1];
         __syncthreads();   // (s_b is reset by the next chunk)
+        }
         for (int b = b0; b <= b1 && b < a.nblocks; ++b) {
-            const int64_t bb = b == 0 ? 0 : end_of(b - 1), be = end_of(b);
+            const int64_t bb = DIRECT || b == 0 ? 0 : end_of(b - 1), be = DIRECT ? mc : end_of(b);
             const int64_t cb = lo > bb ? lo : bb, ce = hi < be ? hi : be;
             if (cb >= ce) continue;
             const int bx = b % a.nbx, by = b / a.nbx;
             const int x0b = bx * BW, y0b = by * BH;   // 0-based first tile of the block
             const int x = x0b + (li & (BW - 1)), y = y0b + (li >> SX);
             const bool in_image = lane < 16 && x < a.ntx && y < a.nty;
-            int32_t* const row = a.table + (k + b) * (int64_t)tpb;
+            BinCount* const row = table + (DIRECT ? k : k + b) * (int64_t)tpb;
             int32_t cnt[16];   // WRITE: the next output index of each tile
             int32_t start = 0;
             int32_t seg_hits = 0;   // WRITE, lane i < 16: this segment's hits of tile i (COUNT's row)
@@ -1091,7 +1112,8 @@ __global__ __launch_bounds__(1024) void k_bin_tiles(BinArgs a) {
                     if (part == 0) seg_hits = row[tl];
                     if (part == 0 && tile > 0) start = a.tiles_end[tile - 1];
 #pragma unroll 4
-                    for (int64_t k2 = bb / nt + part; k2 < k; k2 += 4) start += a.table[(k2 + b) * (int64_t)tpb + tl];
+                    for (int64_t k2 = (DIRECT ? b * cpb : bb / nt) + part; k2 < k; k2 += 4)
+                        start += table[(DIRECT ? k2 : k2 + b) * (int64_t)tpb + tl];
                 }
                 start += __shfl_xor(start, 16);
                 start += __shfl_xor(start, 32);
@@ -1100,7 +1122,7 @@ __global__ __launch_bounds__(1024) void k_bin_tiles(BinArgs a) {
             // masks come sorted along with them (cmask), else from the rectangles.
             int32_t f[PER];
             uint32_t mk[PER];
-            if (a.cmask) {
+            if (!DIRECT && a.cmask) {
 #pragma unroll
                 for (int q = 0; q < PER; ++q) {
                     const int64_t e = cb + t + (int64_t)blockDim.x * q;
@@ -1111,12 +1133,15 @@ __global__ __launch_bounds__(1024) void k_bin_tiles(BinArgs a) {
 #pragma unroll
                 for (int q = 0; q < PER; ++q) {
                     const int64_t e = cb + t + (int64_t)blockDim.x * q;
-                    f[q] = e < ce ? a.cvals[e] : 0;
+                    f[q] = e < ce ? (DIRECT ? a.sorted_f[e] : a.cvals[e]) : 0;
                 }
                 int4 r[PER];
 #pragma unroll
-                for (int q = 0; q < PER; ++q)
-                    r[q] = f[q] > 0 ? reinterpret_cast<const int4*>(a.ranges)[f[q] - 1] : make_int4(1, 1, 0, 0);
+                for (int q = 0; q < PER; ++q) {
+                    const int64_t e = cb + t + (int64_t)blockDim.x * q;
+                    if (DIRECT) r[q] = e < ce ? a.srect[e] : make_int4(1, 1, 0, 0);
+                    else r[q] = f[q] > 0 ? reinterpret_cast<const int4*>(a.ranges)[f[q] - 1] : make_int4(1, 1, 0, 0);
+                }
 #pragma unroll
                 for (int q = 0; q < PER; ++q) {
                     // columns in bits 0-15, rows in bits 16-31 (of the block); none for an empty slot
@@ -1223,7 +1248,7 @@ __global__ __launch_bounds__(1024) void k_bin_tiles(BinArgs a) {
                     const int32_t c = (int32_t)((word >> (16 * ((i >> 1) & 1))) & 0xffffu);
                     mine = lane == i ? c : mine;
                 }
-                if (lane < 16) row[li] = mine;
+                if (lane < 16) row[li] = (BinCount)mine;
                 if (in_image && mine != 0) atomicAdd(&a.tile_totals[x + y * a.ntx], mine);
                 __syncthreads();   // s_f, s_m are free again
                 continue;
@@ -1248,6 +1273,53 @@ __global__ __launch_bounds__(1024) void k_bin_tiles(BinArgs a) {
             __syncthreads();   // s_f, s_m are free again
         }
     }
+}
+
+// Small scenes: whether the tile lists come straight from the depth-ordered Gaussians. The coarse list
+// (count scan, k_emit_count, k_emit_scatter: three launches, 33-35 us at any size below ~100k
+// Gaussians, nearly all of it latency, and more passes still above 255 blocks) exists so that a block
+// of tiles looks only at the Gaussians that reach it; where blocks x Gaussians are few tests anyway,
+// k_bin_tiles<.., DIRECT> tests them all (a Gaussian that misses the block costs its rectangle's read
+// and an empty mask) and k_direct_counts (one workgroup) takes M from the presort's sums. Its cost
+// grows with the tests and, since a chunk sums its block's earlier chunks, with n besides. A frame's
+// us, coarse -> direct, by n blocks (1 + n / 60000): 0.05M (10k, 256x256) 129 -> 94; 0.43M (20k, 400x400)
+// 145 -> 107; 1.5M (50k, 400x400) 148 -> 122; 1.6M (10k, 1080p) 165 -> 128; 2.9M (60k, 979x546, 16x32
+// tiles) 137 -> 102; 3.6M (20k, 1080p) 191 -> 179; 4.8M (60k, 979x546) 157 -> 154 and, half of them out
+// of view, 130 -> 104; 5.8M (120k, 400x400) 157 -> 157; 5.9M (60k, 800x800) 158 -> 168; 6.7M (100k,
+// 600x600) 156 -> 166; 13.9M (200k, 400x400) 162 -> 204. In 8 x 8 tiles at 1080p (16 x 8 blocks): 0.5M
+// (2k) 518 -> 109, 3.0M (10k) 258 -> 182.
+constexpr double kDirectTests = 5.2e6, kDirectChunked = 60000.0;
+static bool direct_lists(int64_t n, const BinGeom& g, int64_t key_cap) {
+    const int64_t nt = (int64_t)g.tpb() * 4 * bin_per(g.sx);
+    return (double)n * g.nblocks() * (1.0 + (double)n / kDirectChunked) <= kDirectTests &&
+           // the count table lies in the key array, four 16-bit counts per key
+           ceil_div(n, nt) * g.nblocks() * g.tpb() <= 4 * key_cap;
+}
+
+// One workgroup: dc[kCntCoarse] = the sum of the presort's packed counts ((M << 32) | coarse entries),
+// with device counts the frame's status (as k_emit_count), and zero[0, nzero) cleared.
+__global__ __launch_bounds__(1024) void k_direct_counts(const int64_t* __restrict__ sums, int64_t nsums, int64_t* dc,
+                                                        int device_counts, int64_t key_cap, int32_t* zero,
+                                                        int64_t nzero) {
+    __shared__ int64_t s_w[1024 / kWave];
+    const int t = threadIdx.x;
+    for (int64_t k = t; k < nzero; k += 1024) zero[k] = 0;
+    int64_t v = 0;
+    for (int64_t k = t; k < nsums; k += 1024) v += sums[k];
+    for (int d = kWave / 2; d >= 1; d >>= 1) v += __shfl_xor(v, d);
+    if (t % kWave == 0) s_w[t / kWave] = v;
+    __syncthreads();
+    if (t != 0) return;
+    int64_t packed = 0;
+    for (int k = 0; k < 1024 / kWave; ++k) packed += s_w[k];
+    dc[kCntCoarse] = packed;
+    if (!device_counts) return;
+    const int64_t keys = packed >> 32;
+    const int64_t st = keys > key_cap ? kFrameKeyCapacity : keys >= (int64_t)INT32_MAX ? kFrameKeyRange : kFrameOk;
+    dc[1] = keys;
+    dc[kCntKeysUsed] = st == kFrameOk ? keys : 0;
+    dc[kCntCoarseUsed] = st == kFrameOk ? (packed & kLow32) : 0;
+    dc[kCntStatus] = st;
 }
 
 // One workgroup: tiles_end = inclusive scan of the tiles' totals, 4096 tiles per step (four
@@ -2259,14 +2331,46 @@ static int bin_tile_lists(hipStream_t s, const tdgs_tiling* tiling, tdgs_render_
     const int64_t nchunks = ceil_div(mb > 0 ? mb : 1, (int64_t)bthreads * per);
     const unsigned bgrid = (unsigned)(nchunks < kBinMaxGrid ? nchunks : kBinMaxGrid);
     const size_t lds = (size_t)bthreads * per * 2 * sizeof(uint32_t);
-    if (bg.sx == 3) k_bin_tiles<3, false><<<bgrid, bthreads, lds, s>>>(ba);
-    else k_bin_tiles<4, false><<<bgrid, bthreads, lds, s>>>(ba);
+    if (bg.sx == 3) k_bin_tiles<3, false, false><<<bgrid, bthreads, lds, s>>>(ba);
+    else k_bin_tiles<4, false, false><<<bgrid, bthreads, lds, s>>>(ba);
     TDGS_LAUNCHED();
     k_bin_scan<<<1, 1024, 0, s>>>(r.tile_totals, tiling->nb_tiles_x * tiling->nb_tiles_y, buf->tiles_end,
                                   dc ? dc + kCntKeysUsed : nullptr, m, d_err);
     TDGS_LAUNCHED();
-    if (bg.sx == 3) k_bin_tiles<3, true><<<bgrid, bthreads, lds, s>>>(ba);
-    else k_bin_tiles<4, true><<<bgrid, bthreads, lds, s>>>(ba);
+    if (bg.sx == 3) k_bin_tiles<3, true, false><<<bgrid, bthreads, lds, s>>>(ba);
+    else k_bin_tiles<4, true, false><<<bgrid, bthreads, lds, s>>>(ba);
+    TDGS_LAUNCHED();
+    return TDGS_OK;
+}
+
+// The same lists straight from the depth-ordered Gaussians (direct_lists; nb: their number, a bound
+// with device counts).
+static int bin_tile_lists_direct(hipStream_t s, const tdgs_tiling* tiling, tdgs_render_buffers* buf,
+                                 const RenderScratch& r, int64_t nb, int64_t m, int64_t* dc, uint32_t* d_err) {
+    StageScope sc(TDGS_STAGE_TILE_RANGES, s);
+    const BinGeom bg = bin_geom(tiling);
+    const int64_t kc = buf->key_capacity;
+    BinArgs ba = {};
+    ba.ntx = tiling->nb_tiles_x; ba.nty = tiling->nb_tiles_y; ba.nbx = bg.nbx; ba.sy = bg.sy;
+    ba.nblocks = bg.nblocks();
+    ba.dmc = dc ? dc + kCntCoarseUsed : nullptr;
+    ba.table = buf->keys; ba.tile_totals = r.tile_totals;
+    ba.tiles_end = buf->tiles_end;
+    ba.out = buf->sorted_values; ba.cap = (int32_t)(kc < INT32_MAX ? kc : INT32_MAX); ba.err = d_err;
+    ba.srect = r.srect; ba.sorted_f = r.sorted_f; ba.nb = nb; ba.dnb = dc ? dc + 4 : nullptr;
+    const unsigned bthreads = 4u << (bg.sx + bg.sy);
+    const int per = bin_per(bg.sx);
+    const int64_t nchunks = ceil_div(nb > 0 ? nb : 1, (int64_t)bthreads * per) * ba.nblocks;
+    const unsigned bgrid = (unsigned)(nchunks < kBinMaxGrid ? nchunks : kBinMaxGrid);
+    const size_t lds = (size_t)bthreads * per * 2 * sizeof(uint32_t);
+    if (bg.sx == 3) k_bin_tiles<3, false, true><<<bgrid, bthreads, lds, s>>>(ba);
+    else k_bin_tiles<4, false, true><<<bgrid, bthreads, lds, s>>>(ba);
+    TDGS_LAUNCHED();
+    k_bin_scan<<<1, 1024, 0, s>>>(r.tile_totals, tiling->nb_tiles_x * tiling->nb_tiles_y, buf->tiles_end,
+                                  dc ? dc + kCntKeysUsed : nullptr, m, d_err);
+    TDGS_LAUNCHED();
+    if (bg.sx == 3) k_bin_tiles<3, true, true><<<bgrid, bthreads, lds, s>>>(ba);
+    else k_bin_tiles<4, true, true><<<bgrid, bthreads, lds, s>>>(ba);
     TDGS_LAUNCHED();
     return TDGS_OK;
 }
@@ -2519,7 +2623,13 @@ int tdgs_render(tdgs_ctx* ctx, void* stream, const tdgs_gaussians* g, const tdgs
         // 5: tiles and blocks touched, in depth order -> the blocks' entries (emission offsets)
         // and M (the scan's tile sums come from the depth sort)
         const BinGeom bg = bin_geom(tiling);
-        {
+        const bool direct = direct_lists(n, bg, buf->key_capacity);
+        if (direct) {
+            StageScope sc(TDGS_STAGE_COUNT_SCAN, s);
+            k_direct_counts<<<1, 1024, 0, s>>>(r.scan_sums, ceil_div(n, kScanTile), ctx->d_counters, device_counts,
+                                               buf->key_capacity, r.tile_totals, r.ntt);
+            TDGS_LAUNCHED();
+        } else {
             StageScope sc(TDGS_STAGE_COUNT_SCAN, s);
             const SortedTileBlockCounts stb{r.srect, bg.sx, bg.sy, d_nb};
             TDGS_TRY(device_scan_apply(stb, WriteBlockScan{WriteScanAndBlocks{cs, blk_first, nblk}}, n, r.scan_sums,
@@ -2527,7 +2637,8 @@ int tdgs_render(tdgs_ctx* ctx, void* stream, const tdgs_gaussians* g, const tdgs
         }
         if (device_counts) {
             // 6-8 sized by the key capacity; the blend copies the counts to the frame counts
-            TDGS_TRY(bin_tile_lists(s, tiling, buf, r, n, buf->key_capacity, 0, ctx->d_counters, d_err));
+            if (direct) TDGS_TRY(bin_tile_lists_direct(s, tiling, buf, r, n, 0, ctx->d_counters, d_err));
+            else TDGS_TRY(bin_tile_lists(s, tiling, buf, r, n, buf->key_capacity, 0, ctx->d_counters, d_err));
             StageScope sc(TDGS_STAGE_BLEND, s);
             return launch_render_tiles(s, cam, tiling, opt, buf->key_capacity, buf->tiles_end, buf->sorted_values,
                                        buf->f2d, buf->depths, out, nullptr, ctx->d_counters, frame_counts(buf),
@@ -2549,8 +2660,9 @@ int tdgs_render(tdgs_ctx* ctx, void* stream, const tdgs_gaussians* g, const tdgs
             set_error("key buffers hold %lld keys, %lld needed", (long long)buf->key_capacity, (long long)m);
             return TDGS_ERR_CAPACITY;
         }
-        // 6-8: the tile lists by coarse binning
-        TDGS_TRY(bin_tile_lists(s, tiling, buf, r, nb, mc, m, nullptr, d_err));
+        // 6-8: the tile lists by coarse binning, or directly
+        if (direct) TDGS_TRY(bin_tile_lists_direct(s, tiling, buf, r, nb, m, nullptr, d_err));
+        else TDGS_TRY(bin_tile_lists(s, tiling, buf, r, nb, mc, m, nullptr, d_err));
         // 9: blending
         StageScope sc(TDGS_STAGE_BLEND, s);
         return launch_render_tiles(s, cam, tiling, opt, m, buf->tiles_end, buf->sorted_values, buf->f2d,
