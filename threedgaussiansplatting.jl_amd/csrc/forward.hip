@@ -980,7 +980,10 @@ inline int64_t bin_table_entries(int64_t kc, const BinGeom& g) {
 struct BinArgs {
     int32_t ntx, nty, nbx, sy, nblocks;
     const int32_t* cvals;      // the blocks' lists: fgidx (1-based), block by block, depth order within
-    const int32_t* cend;       // end (exclusive) of each block's run in cvals, or null:
+    union {
+        const int32_t* cend;   // end (exclusive) of each block's run in cvals, or null:
+        const int64_t* dnb;    // (DIRECT)
+    };
     const uint32_t* totals;    // the coarse radix pass's digit totals (block b has id b + 1)
     int64_t mc;                // entries of cvals (launch bound)
     const int64_t* dmc;        // entries used (device counts), or null
@@ -992,12 +995,10 @@ struct BinArgs {
     int32_t* out;              // WRITE: sdfgidx_to_fgidx
     int32_t cap;               // WRITE: entries of out
     uint32_t* err;
-    // DIRECT: every block's candidates are all non-empty Gaussians in depth order
-    const int4* srect;         // their rectangles
-    const int32_t* sorted_f;   // and fgidx
-    int64_t nb;                // how many (launch bound)
-    const int64_t* dnb;        // how many (device counts), or null
 };
+// DIRECT: every block's candidates are all non-empty Gaussians in depth order. cvals holds their fgidx, ranges
+// their rectangles in that order, mc their number (launch bound); dnb (device counts), or null, points at it.
+// (The same fields: more of them cost the other variant scalar registers, 17 spilled against 2.)
 
 // Workgroup: 4 threads per tile of a block of 2^SX x 2^sy tiles; wavefront w takes the
 // block's tiles 16 w .. 16 w + 15 (row-major, 2^SX per row). A segment's Gaussians go
@@ -1027,7 +1028,7 @@ __global__ __launch_bounds__(1024) void k_bin_tiles(BinArgs a) {
     BinCount* const table = static_cast<BinCount*>(a.table);
     const int t = threadIdx.x, lane = __lane_id(), w = t / kWave;
     const int nt = (int)blockDim.x * PER;   // entries per chunk
-    int64_t mc = DIRECT ? a.nb : a.mc;
+    int64_t mc = a.mc;
     if (DIRECT && a.dnb && *a.dnb < mc) mc = *a.dnb;
     if (a.dmc && (DIRECT ? *a.dmc == 0 : *a.dmc < mc)) mc = DIRECT ? 0 : *a.dmc;
     const int64_t cpb = (mc + nt - 1) / nt;   // DIRECT: chunks per block
@@ -1133,13 +1134,13 @@ __global__ __launch_bounds__(1024) void k_bin_tiles(BinArgs a) {
 #pragma unroll
                 for (int q = 0; q < PER; ++q) {
                     const int64_t e = cb + t + (int64_t)blockDim.x * q;
-                    f[q] = e < ce ? (DIRECT ? a.sorted_f[e] : a.cvals[e]) : 0;
+                    f[q] = e < ce ? a.cvals[e] : 0;
                 }
                 int4 r[PER];
 #pragma unroll
                 for (int q = 0; q < PER; ++q) {
                     const int64_t e = cb + t + (int64_t)blockDim.x * q;
-                    if (DIRECT) r[q] = e < ce ? a.srect[e] : make_int4(1, 1, 0, 0);
+                    if (DIRECT) r[q] = e < ce ? reinterpret_cast<const int4*>(a.ranges)[e] : make_int4(1, 1, 0, 0);
                     else r[q] = f[q] > 0 ? reinterpret_cast<const int4*>(a.ranges)[f[q] - 1] : make_int4(1, 1, 0, 0);
                 }
 #pragma unroll
@@ -2357,7 +2358,8 @@ static int bin_tile_lists_direct(hipStream_t s, const tdgs_tiling* tiling, tdgs_
     ba.table = buf->keys; ba.tile_totals = r.tile_totals;
     ba.tiles_end = buf->tiles_end;
     ba.out = buf->sorted_values; ba.cap = (int32_t)(kc < INT32_MAX ? kc : INT32_MAX); ba.err = d_err;
-    ba.srect = r.srect; ba.sorted_f = r.sorted_f; ba.nb = nb; ba.dnb = dc ? dc + 4 : nullptr;
+    ba.cvals = r.sorted_f; ba.ranges = reinterpret_cast<const int32_t*>(r.srect); ba.mc = nb;
+    ba.dnb = dc ? dc + 4 : nullptr;
     const unsigned bthreads = 4u << (bg.sx + bg.sy);
     const int per = bin_per(bg.sx);
     const int64_t nchunks = ceil_div(nb > 0 ? nb : 1, (int64_t)bthreads * per) * ba.nblocks;

@@ -64,25 +64,25 @@ inline float exponent_cut(float min_alpha) {
 }
 
 // The exponent from which alpha = exp_f(e) reaches min_alpha: exp_f(e) >= min_alpha exactly for e >= *cut.
-// Around a min_alpha of at most 0.9 neighbouring exponents are at least 7e-9 apart and exp_f is within
-// 0.91 ulp (1.1e-7) of a strictly rising function, so the switch is looked for within 32 floats of
-// log(min_alpha) and has to be a clean one there (further away the order is certain). False when there
-// is none, when max_alpha stays below min_alpha, or when *cut < -80 (results of exp_f near its
-// flush to zero).
+// exp_f is within 0.91 ulp (1.1e-7 relative) of a strictly rising function and neighbouring exponents of
+// at least 1 in size lie 1.2e-7 apart or more, so there the switch is at most two floats from
+// log(min_alpha) rounded and is looked for within four; within 32 up to a min_alpha of 0.9, where
+// the exponents lie at least 7e-9 apart. It has to be a clean one. (Each look costs the host ~40 ns, which a
+// frame with host counts waits for.) False when there is none, when max_alpha stays below min_alpha,
+// or when *cut < -80 (results of exp_f near its flush to zero).
 inline bool exact_exponent_cut(float min_alpha, float max_alpha, float* cut) {
     *cut = 0.0f;
     if (!(min_alpha > 0.0f) || !(min_alpha <= 0.9f) || !(max_alpha >= min_alpha)) return false;
-    constexpr int kSpan = 32;
-    float e = (float)std::log((double)min_alpha);
-    if (!(e >= -80.0f)) return false;
-    for (int k = 0; k < kSpan; ++k) e = std::nextafter(e, -kInf);
+    const float mid = (float)std::log((double)min_alpha);   // negative: one float up is one less in the bits
+    if (!(mid >= -80.0f)) return false;
+    const int span = mid <= -1.0f ? 4 : 32;
     bool reached = false;
-    for (int k = 0; k < 2 * kSpan; ++k, e = std::nextafter(e, kInf)) {
+    for (int k = -span; k < span; ++k) {
+        const float e = bits_float(float_bits(mid) - (uint32_t)k);
         const bool r = exp_f(e) >= min_alpha;
+        if (r ? k == -span : reached) return false;
         if (r && !reached) *cut = e;
-        if (!r && reached) return false;
         reached = r;
-        if (r && k == 0) return false;
     }
     return reached;
 }
