@@ -1007,19 +1007,23 @@ struct BinArgs {
 // counters over its own candidates, summed over the wavefront; WRITE tests 64 candidates at a
 // time against a tile with one ballot and writes each hit at the tile's list start + the
 // earlier segments' hits + the hits before it.
-// (Staging the writes in LDS rings and storing 64 entries at a time measured no faster.)
-// LDS (dynamic): the chunk's candidates, 2 bin_per(SX) words per thread.
+// LDS (dynamic): the chunk's candidates, bin_per(SX) masks per thread (COUNT) or as many pairs of fgidx
+// and mask (WRITE: one 8-byte read).
 // DIRECT (small scenes): no coarse list. Chunk k = b cpb + c tests the c-th run of nt of all
 // Gaussians against block b (cpb = ceil(N_b / nt)), the masks made from the contiguous depth-ordered
 // rectangles; its counts are table[k tpb + local tile]. See direct_lists.
+// (lane_rank: base plus the set bits of bal below the lane's.)
+__device__ __forceinline__ uint32_t lane_rank(uint64_t bal, int32_t base = 0) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, (uint32_t)base));
+}
 template <int SX, bool WRITE, bool DIRECT>
 __global__ __launch_bounds__(1024) void k_bin_tiles(BinArgs a) {
-    extern __shared__ uint32_t s_dyn[];
+    extern __shared__ __align__(8) uint32_t s_dyn[];
     __shared__ int32_t s_cend[1024];   // the blocks' ends, when there are at most 1024 blocks
     __shared__ int32_t s_b[2];
     constexpr int PER = bin_per(SX);
-    int32_t* const s_f = reinterpret_cast<int32_t*>(s_dyn);   // the candidates' fgidx
-    uint32_t* const s_m = s_dyn + blockDim.x * PER;           // and tile masks
+    uint2* const s_fm = reinterpret_cast<uint2*>(s_dyn);   // WRITE: the candidates' fgidx and tile masks
+    uint32_t* const s_m = s_dyn;                           // COUNT: their tile masks
     constexpr int BW = 1 << SX;
     const int BH = 1 << a.sy;
     const int tpb = BW * BH;
@@ -1155,8 +1159,8 @@ __global__ __launch_bounds__(1024) void k_bin_tiles(BinArgs a) {
             }
 #pragma unroll
             for (int q = 0; q < PER; ++q) {
-                s_f[t + blockDim.x * q] = f[q];
-                s_m[t + blockDim.x * q] = mk[q];
+                if (WRITE) s_fm[t + blockDim.x * q] = make_uint2((uint32_t)f[q], mk[q]);
+                else s_m[t + blockDim.x * q] = mk[q];
             }
             __syncthreads();
             const int nk = __builtin_amdgcn_readfirstlane((int)(ce - cb));
@@ -1174,7 +1178,13 @@ __global__ __launch_bounds__(1024) void k_bin_tiles(BinArgs a) {
             // per 64 candidates for all 16 tiles). (At 3840 x 2160, 3M Gaussians, runs average
             // ~1100 entries: lists 1.31 -> 0.92 ms; at 1920 x 1080, 1M Gaussians, ~70, and the
             // tile-major walk from 16 hits per 64 candidates alone measured 45 -> 49 us.)
-            if (WRITE && wave_hits >= 4 * nk && wave_hits >= 16 * 256) {
+            // It also takes what the candidate-major loop does not: a frame whose keys do not fit (an index
+            // past a.cap - 1 is clamped; the frame is thrown away) and lists past 32-bit byte offsets.
+            // (752M keys, 3.0 GB, at 3840 x 2160: 4.1 TB/s of writes, and no faster with half the
+            // instructions, with full aligned 1 KB stores through an LDS ring, or with chunks twice as
+            // long; non-temporal stores double the time. Memory it is.)
+            const bool fits = WRITE && __ballot(lane < 16 && start + seg_hits > min(a.cap, 1 << 30)) == 0;
+            if (WRITE && (!fits || (wave_hits >= 4 * nk && wave_hits >= 16 * 256))) {
                 const int row0 = 16 + __builtin_amdgcn_readfirstlane(ly0);
 #pragma unroll 1
                 for (int i = 0; i < 16; ++i) {
@@ -1184,27 +1194,15 @@ __global__ __launch_bounds__(1024) void k_bin_tiles(BinArgs a) {
                     int32_t c = __builtin_amdgcn_readlane(start, i);
                     const int32_t c_end = c + nh;
                     // (entries past nk are zero: no hits)
-                    int32_t nf = s_f[lane];
-                    uint32_t nm = s_m[lane];
                     for (int j0 = 0; j0 < nk && c < c_end; j0 += kWave) {
-                        const int32_t fv = nf;
-                        const uint32_t p = nm;
-                        if (j0 + kWave < nk) {   // read ahead, both words
-                            nf = s_f[j0 + kWave + lane];
-                            nm = s_m[j0 + kWave + lane];
-                        }
-                        asm volatile("" ::"v"(fv));   // not sunk into the branch below
-                        const bool hit = (p & need) == need;
-                        const uint64_t bal = __ballot(hit);
-                        if (hit) {
-                            const int32_t o = (int32_t)__builtin_amdgcn_mbcnt_hi(
-                                (uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, (uint32_t)c));
-                            a.out[o < a.cap ? o : a.cap - 1] = fv;
-                        }
+                        const uint2 fm = s_fm[j0 + lane];
+                        const uint64_t bal = __ballot((fm.y & need) == need);
+                        if (__builtin_amdgcn_inverse_ballot_w64(bal))
+                            a.out[min((int32_t)lane_rank(bal, c), a.cap - 1)] = (int32_t)fm.x;
                         c += __popcll(bal);
                     }
                 }
-                __syncthreads();   // s_f, s_m are free again
+                __syncthreads();   // s_fm is free again
                 continue;
             }
 #pragma unroll
@@ -1251,27 +1249,27 @@ __global__ __launch_bounds__(1024) void k_bin_tiles(BinArgs a) {
                 }
                 if (lane < 16) row[li] = (BinCount)mine;
                 if (in_image && mine != 0) atomicAdd(&a.tile_totals[x + y * a.ntx], mine);
-                __syncthreads();   // s_f, s_m are free again
+                __syncthreads();   // s_m is free again
                 continue;
             }
+            // Bound by instruction issue: 6 vector ones and the store per tile and 64 candidates (a mask
+            // compare that is itself the store's predicate, no clamp, a 32-bit offset to a scalar base).
+            // 1M Gaussians, 1080p: 27.1 us with 11 of them (two compares, a clamp, a 64-bit address), 21.5 now.
             for (int j0 = 0; j0 < nk; j0 += kWave) {
-                const uint32_t h = tile_bits(s_m[j0 + lane]);   // (entries past nk are zero: no hits)
-                const int32_t fv = s_f[j0 + lane];
+                const uint2 c = s_fm[j0 + lane];
+                const uint32_t h = tile_bits(c.y);   // (entries past nk are zero: no hits)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
-                    const bool hit = (h >> i) & 1u;
-                    const uint64_t bal = __ballot(hit);
-                    if (hit) {
-                        // the tile's next index plus the hits in lower lanes (v_mbcnt); the
-                        // counts come from the same walk, the index is clamped all the same
-                        const int32_t o = (int32_t)__builtin_amdgcn_mbcnt_hi(
-                            (uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, (uint32_t)cnt[i]));
-                        a.out[o < a.cap ? o : a.cap - 1] = fv;
+                    const uint64_t bal = __ballot((h & (1u << i)) != 0);
+                    if (__builtin_amdgcn_inverse_ballot_w64(bal)) {
+                        // the tile's next index plus the hits in lower lanes, as a byte offset of 32 bits
+                        const uint32_t o = lane_rank(bal, cnt[i]);
+                        *reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(a.out) + 4 * o) = c.x;
                     }
                     cnt[i] += __popcll(bal);
                 }
             }
-            __syncthreads();   // s_f, s_m are free again
+            __syncthreads();   // s_fm is free again
         }
     }
 }
@@ -2331,15 +2329,15 @@ static int bin_tile_lists(hipStream_t s, const tdgs_tiling* tiling, tdgs_render_
     const int per = bin_per(bg.sx);
     const int64_t nchunks = ceil_div(mb > 0 ? mb : 1, (int64_t)bthreads * per);
     const unsigned bgrid = (unsigned)(nchunks < kBinMaxGrid ? nchunks : kBinMaxGrid);
-    const size_t lds = (size_t)bthreads * per * 2 * sizeof(uint32_t);
+    const size_t lds = (size_t)bthreads * per * sizeof(uint32_t);   // COUNT's; WRITE's is twice that
     if (bg.sx == 3) k_bin_tiles<3, false, false><<<bgrid, bthreads, lds, s>>>(ba);
     else k_bin_tiles<4, false, false><<<bgrid, bthreads, lds, s>>>(ba);
     TDGS_LAUNCHED();
     k_bin_scan<<<1, 1024, 0, s>>>(r.tile_totals, tiling->nb_tiles_x * tiling->nb_tiles_y, buf->tiles_end,
                                   dc ? dc + kCntKeysUsed : nullptr, m, d_err);
     TDGS_LAUNCHED();
-    if (bg.sx == 3) k_bin_tiles<3, true, false><<<bgrid, bthreads, lds, s>>>(ba);
-    else k_bin_tiles<4, true, false><<<bgrid, bthreads, lds, s>>>(ba);
+    if (bg.sx == 3) k_bin_tiles<3, true, false><<<bgrid, bthreads, 2 * lds, s>>>(ba);
+    else k_bin_tiles<4, true, false><<<bgrid, bthreads, 2 * lds, s>>>(ba);
     TDGS_LAUNCHED();
     return TDGS_OK;
 }
@@ -2364,15 +2362,15 @@ static int bin_tile_lists_direct(hipStream_t s, const tdgs_tiling* tiling, tdgs_
     const int per = bin_per(bg.sx);
     const int64_t nchunks = ceil_div(nb > 0 ? nb : 1, (int64_t)bthreads * per) * ba.nblocks;
     const unsigned bgrid = (unsigned)(nchunks < kBinMaxGrid ? nchunks : kBinMaxGrid);
-    const size_t lds = (size_t)bthreads * per * 2 * sizeof(uint32_t);
+    const size_t lds = (size_t)bthreads * per * sizeof(uint32_t);   // COUNT's; WRITE's is twice that
     if (bg.sx == 3) k_bin_tiles<3, false, true><<<bgrid, bthreads, lds, s>>>(ba);
     else k_bin_tiles<4, false, true><<<bgrid, bthreads, lds, s>>>(ba);
     TDGS_LAUNCHED();
     k_bin_scan<<<1, 1024, 0, s>>>(r.tile_totals, tiling->nb_tiles_x * tiling->nb_tiles_y, buf->tiles_end,
                                   dc ? dc + kCntKeysUsed : nullptr, m, d_err);
     TDGS_LAUNCHED();
-    if (bg.sx == 3) k_bin_tiles<3, true, true><<<bgrid, bthreads, lds, s>>>(ba);
-    else k_bin_tiles<4, true, true><<<bgrid, bthreads, lds, s>>>(ba);
+    if (bg.sx == 3) k_bin_tiles<3, true, true><<<bgrid, bthreads, 2 * lds, s>>>(ba);
+    else k_bin_tiles<4, true, true><<<bgrid, bthreads, 2 * lds, s>>>(ba);
     TDGS_LAUNCHED();
     return TDGS_OK;
 }
