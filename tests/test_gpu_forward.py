@@ -64,6 +64,21 @@ def test_render_helpers_known_answers(gpu):
     assert te.cpu().tolist() == gold["tiles_end"]
 
 
+@pytest.mark.parametrize("n", [4096, 512 * 4096, 512 * 4096 + 1])   # the grouped tables' last tile, and past it
+@pytest.mark.parametrize("digits", [1, 2, 200])
+def test_sort_pairs_equal_digits(gpu, n, digits):
+    """Wavefronts whose keys share a digit, or nearly: a few different keys, one odd key among them."""
+    rng = np.random.default_rng(n + digits)
+    keys = rng.integers(0, digits, size=n).astype(np.int64) * 0x0101_0101_0101_0101
+    keys[n // 3] = 0x7f00_ff00_ff00_ff00
+    vals = np.arange(n, dtype=np.int32)
+    order = np.argsort(keys.view(np.uint64), kind="stable")
+    dev = torch.device("cuda", 0)
+    gk, gv = gpu.sort_pairs(torch.from_numpy(keys).to(dev), torch.from_numpy(vals).to(dev), 64)
+    np.testing.assert_array_equal(gv.cpu().numpy(), vals[order])
+    np.testing.assert_array_equal(gk.cpu().numpy(), keys[order])
+
+
 @pytest.mark.parametrize("n,end_bit,spread", [(1, 41, 4), (1000, 41, 8), (4097, 45, 16), (100_000, 45, 64),
                                               (300_000, 64, 1 << 40), (70_000, 20, 1000),
                                               (2_000_000, 46, 5000), (600_000, 40, 1)])

@@ -298,8 +298,7 @@ __global__ __launch_bounds__(kRsThreads) void k_ds_count(const uint32_t* __restr
         const bool valid = key[j] != 0xffffffffu;
         const uint32_t d = valid ? (uint32_t)ds_bucket(((uint64_t)key[j] << 32) | (uint64_t)(i + 1), s_spl) : 0u;
         if (i < n) bid[i] = (uint8_t)d;
-        const uint64_t peers = match_digit(d, 8, valid);
-        if (valid && (peers & lanemask_lt()) == 0) atomicAdd(&s_h[d], (uint32_t)__popcll(peers));
+        count_digit(s_h, d, valid);
     }
     __syncthreads();
     if (t < kRsBins) {

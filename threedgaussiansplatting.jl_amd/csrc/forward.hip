@@ -2465,11 +2465,18 @@ int tdgs_emit_keys(void* stream, int32_t nb_fgaussians, const float* depths, con
     return TDGS_OK;
 }
 
+// Group sums of the grouped passes: for any end_bit, and of as many tiles as those take (the scratch
+// never shrinks as n grows).
+static int64_t sort_pairs_group_words(int64_t n) {
+    const int64_t most = RsTile<uint64_t>::kGroupedTiles * RsTile<uint64_t>::kTile;
+    return radix_group_words<uint64_t>(n < most ? n : most, 0, 64);
+}
+
 size_t tdgs_sort_pairs_temp_bytes(int32_t n, int32_t end_bit) {
     (void)end_bit;
     const int64_t nn = n > 0 ? n : 1;
     return align_up((size_t)nn * sizeof(int64_t)) + align_up((size_t)nn * sizeof(int32_t)) +
-           radix_temp_bytes(nn);
+           align_up(radix_temp_bytes(nn)) + (size_t)sort_pairs_group_words(nn) * sizeof(uint32_t);
 }
 
 int tdgs_sort_pairs(void* temp, size_t temp_bytes, const int64_t* keys_in, int64_t* keys_out,
@@ -2485,8 +2492,18 @@ int tdgs_sort_pairs(void* temp, size_t temp_bytes, const int64_t* keys_in, int64
     int32_t* alt_v = ar.take<int32_t>(n);
     const size_t rb = radix_temp_bytes(n);
     void* rtemp = ar.take<char>((int64_t)rb);
-    return radix_sort_pairs<uint64_t>((const uint64_t*)keys_in, (uint64_t*)keys_out, values_in, values_out,
-                                      alt_k, alt_v, n, 0, end_bit, rtemp, rb, (hipStream_t)stream);
+    uint32_t* grp = nullptr;
+    int64_t words = 0;
+    if (radix_tiles<uint64_t>(n) <= RsTile<uint64_t>::kGroupedTiles) {
+        words = radix_group_words<uint64_t>(n, 0, end_bit);
+        grp = ar.take<uint32_t>(words);
+        if (grp && words > 0) {
+            k_fill_i32<<<(unsigned)ceil_div(words, 256), 256, 0, (hipStream_t)stream>>>((int32_t*)grp, words, 0);
+            TDGS_LAUNCHED();
+        }
+    }
+    return radix_sort_pairs_grouped<uint64_t>((const uint64_t*)keys_in, (uint64_t*)keys_out, values_in, values_out,
+                                              alt_k, alt_v, n, 0, end_bit, rtemp, rb, grp, words, (hipStream_t)stream);
 }
 
 int tdgs_tile_ranges(void* stream, int64_t nb_keys, const int64_t* sorted_keys, int32_t nb_tiles,

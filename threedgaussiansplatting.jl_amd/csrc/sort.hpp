@@ -15,7 +15,7 @@
 // The count of a pass can come from the kernel that produced the keys (the render pipeline
 // fuses it into key emission), so a pass reads its keys once.
 //
-// Grouped variant (radix_sort_pairs_grouped, up to kRsMaxGroupedTiles tiles): two launches a
+// Grouped variant (radix_sort_pairs_grouped, up to RsTile::kGroupedTiles tiles): two launches a
 // pass. The count writes each tile's histogram as one contiguous row (cnt[tile][digit]) and
 // adds it into the sums of its group of kRsGroup tiles (grp[group][digit], 16 atomics per
 // word); each scatter workgroup then finds its own offsets by summing the earlier groups'
@@ -38,10 +38,16 @@ constexpr int kRsBins = 256;
 // Keys per thread and per tile (4096-key tiles). 8192-key tiles for the 64-bit keys (twice
 // the keys per digit per tile, so twice-as-long output runs) measured 6% faster on 751M keys
 // but 35% slower on 6M keys (half the workgroups, at 151 VGPRs and 74 KB of LDS each).
+// kGroupedTiles: the most tiles radix_sort_pairs_grouped sorts with grouped tables. A scatter workgroup
+// reads every group's sums (16 tiles each), so their cost per pass grows with the square of the tiles,
+// and a scan launch takes 5 us at any size: 64-bit pairs of 45 bits, grouped against row scans, 118 vs
+// 137 us at 1M, 148 vs ~152 at 2M, 182 vs 175 at 3M, 391 vs 324 at 6.15M; the presort's 32-bit keys 80
+// vs 86 us at 1.5M, 96 vs 98 at 2M, 172 vs 139 at 3M, 322 vs 198 at 6M.
 template <class K>
 struct RsTile {
     static constexpr int kItems = 8;
     static constexpr int kTile = kRsThreads * kItems;
+    static constexpr int64_t kGroupedTiles = 512;
 };
 // 32-bit keys are the depth presort's: ~1M keys of which the later passes sort the few
 // hundred thousand non-empty ones. 2048-key tiles spread them over more CUs (72 us vs 81 us
@@ -50,6 +56,7 @@ template <>
 struct RsTile<uint32_t> {
     static constexpr int kItems = 4;
     static constexpr int kTile = kRsThreads * kItems;
+    static constexpr int64_t kGroupedTiles = 1024;
 };
 constexpr int kRsMinTile = kRsThreads * 4;   // the smallest tile above (sizes the count table)
 static_assert(RsTile<uint16_t>::kTile >= kRsMinTile && RsTile<uint32_t>::kTile >= kRsMinTile &&
@@ -100,8 +107,23 @@ __device__ __forceinline__ uint32_t digit_excl_scan(uint32_t a, uint32_t* s_tmp)
     return off + ia - a;
 }
 
-// Histogram of one digit over a tile into LDS (wave-aggregated atomics); returns after a
-// block barrier with s_h complete.
+// Adds the wavefront's digits to s_h (lanes with valid; every lane of the wavefront calls it): one
+// LDS atomic per key, or one in all where every lane holds the same digit (the top digits of
+// depths). Lanes of one digit serialise in the LDS unit, but even 64 of them cost about what
+// finding the equal lanes first did (8 ballots and some 40 vector instructions per 64 keys): a
+// count of 6.15M 64-bit keys 17.6 -> 9.6 us, of one, two or four different keys no slower than before.
+__device__ __forceinline__ void count_digit(uint32_t* s_h, uint32_t d, bool valid) {
+    const uint64_t in = __ballot(valid);
+    if (in == 0) return;
+    const uint32_t d0 = (uint32_t)__builtin_amdgcn_readlane((int)d, __builtin_ctzll(in));
+    if (__ballot(valid && d != d0) == 0) {
+        if (__lane_id() == 0) atomicAdd(&s_h[d0], (uint32_t)__popcll(in));
+    } else if (valid) {
+        atomicAdd(&s_h[d], 1u);
+    }
+}
+
+// Histogram of one digit over a tile into LDS; returns after a block barrier with s_h complete.
 template <class K>
 __device__ __forceinline__ void tile_digit_histogram(const K* __restrict__ keys, int64_t n, int64_t tile, int shift,
                                                      int nbits, uint32_t* s_h, bool drop_max = false) {
@@ -121,8 +143,7 @@ __device__ __forceinline__ void tile_digit_histogram(const K* __restrict__ keys,
     for (int k = 0; k < kRsItems; ++k) {
         const bool valid = base + (int64_t)k * kRsThreads < n && !(drop_max && key[k] == (K)~(K)0);
         const uint32_t d = (uint32_t)(key[k] >> shift) & mask;
-        const uint64_t peers = match_digit(d, nbits, valid);
-        if (valid && (peers & lanemask_lt()) == 0) atomicAdd(&s_h[d], (uint32_t)__popcll(peers));
+        count_digit(s_h, d, valid);
     }
     __syncthreads();
 }
@@ -637,7 +658,7 @@ inline int64_t radix_group_words(int64_t n, int begin_bit, int end_bit) {
 // radix_sort_pairs (same arguments, without first_counts) with the grouped count tables: a
 // count and a scatter launch per pass. zgrp holds radix_group_words<K>(n, ...) words that are
 // zero on entry (an earlier launch on the stream clears them); they hold the group sums after.
-// Sorts of more than kRsMaxGroupedTiles tiles, or with too few words in zgrp, take
+// Sorts of more than RsTile<K>::kGroupedTiles tiles, or with too few words in zgrp, take
 // radix_sort_pairs' path (zgrp unused).
 template <class K>
 int radix_sort_pairs_grouped(const K* kin, K* kout, const int32_t* vin, int32_t* vout, K* alt_k, int32_t* alt_v,
@@ -649,7 +670,7 @@ int radix_sort_pairs_grouped(const K* kin, K* kout, const int32_t* vin, int32_t*
     const int64_t tiles = radix_tiles<K>(n);
     const int64_t gwords = rs_groups(tiles) * kRsBins;
     if (n <= 0) return TDGS_OK;
-    if (passes == 0 || n > (int64_t)INT32_MAX || tiles > kRsMaxGroupedTiles || zgrp == nullptr ||
+    if (passes == 0 || n > (int64_t)INT32_MAX || tiles > RsTile<K>::kGroupedTiles || zgrp == nullptr ||
         zgrp_words < passes * gwords)
         return radix_sort_pairs<K>(kin, kout, vin, vout, alt_k, alt_v, n, begin_bit, end_bit, temp, temp_bytes,
                                    stream, nullptr, err, kept_out, d_count, gather);
