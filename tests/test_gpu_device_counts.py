@@ -282,3 +282,25 @@ def test_small_scene_lists_match_oracle(gpu, oracle, n, w, h, tile):
         assert (nbf, m, status) == (r["nb_fgaussians"], r["nb_keys"], abi.TDGS_FRAME_KEY_CAPACITY)
         assert float(out.T.min()) == 1.0 and int(out.last.max()) == 0
     gpu.ctx_check(0)
+
+
+@pytest.mark.parametrize("n", [33_026, 66_060])   # just past 2^31 keys, and past 2^32
+def test_more_keys_than_indices(gpu, n):
+    """Frames whose M does not fit 32 bits, signed or not: refused with the exact M on the host, a void
+    frame with the exact M and a status on the device."""
+    cam = host.look_at_camera(1020, 1020, 60.0, (0.0, 0.0, -4.0))
+    t = host.Tiling.for_camera(cam, 4, 4)   # 65025 tiles
+    opts = host.RenderOptions.for_camera(cam, 0)
+    g_host = synthetic.config(0, n=n).gaussians
+    g_host.means_opacity[:] = 0.0
+    g_host.scaling[:] = 3.0   # (every Gaussian covers the image)
+    g = gpu.TrainableGaussiansVector.from_host(g_host, 0)
+    out, buf = _device_render(gpu, g, cam, t, opts, key_capacity=100_000)
+    m = int(buf.counts[:n].sum(dtype=torch.int64))
+    assert m == n * 65025
+    assert buf.frame_counts() == (n, m, n, abi.TDGS_FRAME_KEY_CAPACITY)
+    assert float(out.T.min()) == 1.0 and int(out.last.max()) == 0
+    assert _monitor(gpu)[3] == m
+    with pytest.raises(gpu.CapacityError, match=f"{m} duplicated keys exceed"):
+        gpu.render_(out, g, cam, t, opts, buf)
+    gpu.ctx_check(0)

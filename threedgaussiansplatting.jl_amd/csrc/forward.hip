@@ -655,12 +655,10 @@ __global__ __launch_bounds__(kEmitSortThreads) void k_emit_count(int64_t nb, int
         // device counts: the grid covers key_cap entries; when the M keys fit the key arrays the
         // passes emit the blocks' entries (at most M), else none (the status says why)
         nb = dc[4];
-        const int64_t packed = dc[kCntCoarse];   // (M << 32) | coarse entries, from the scan
-        const int64_t keys = packed >> 32;
+        const int64_t keys = dc[1];   // M, from the scan
         const int64_t st = keys > key_cap ? kFrameKeyCapacity : keys >= (int64_t)INT32_MAX ? kFrameKeyRange : kFrameOk;
-        m = st == kFrameOk ? (packed & kLow32) : 0;
+        m = st == kFrameOk ? dc[kCntCoarse] : 0;
         if (blockIdx.x == 0 && t == 0) {
-            dc[1] = keys;
             dc[kCntKeysUsed] = st == kFrameOk ? keys : 0;
             dc[kCntCoarseUsed] = m;
             dc[kCntStatus] = st;
@@ -929,27 +927,18 @@ static BinGeom bin_geom(const tdgs_tiling* t) {
     return g;
 }
 
-// Tiles and blocks touched by each non-empty Gaussian in depth order, packed as
-// (tiles << 32) | blocks (entries past N_b count 0): one scan gives the blocks' emission
-// offsets in the low half and, in its total, the key count M in the high half (both below
-// 2^31, so the halves never carry into each other).
-struct SortedTileBlockCounts {
+// Blocks touched by each non-empty Gaussian in depth order (entries past N_b count 0), whose scan
+// gives the blocks' emission offsets. The presort's sums of every scan tile hold the tiles touched
+// above the blocks ((tiles << 32) | blocks, at most 2048 x 65535 tiles), so the scan's tile 0 adds up
+// the key count M as well.
+struct SortedBlockCounts {
     const int4* srect;   // rectangles in depth order
     int sx, sy;
     const int64_t* d_nb;
-    __device__ int64_t operator()(int64_t j) const {
+    __device__ int32_t operator()(int64_t j) const {
         if (j >= *d_nb) return 0;
         const int4 r = srect[j];
-        const int32_t blocks =
-            (((r.z - 1) >> sx) - ((r.x - 1) >> sx) + 1) * (((r.w - 1) >> sy) - ((r.y - 1) >> sy) + 1);
-        return ((int64_t)rect_area(r) << 32) | (int64_t)blocks;
-    }
-};
-// WriteScanAndBlocks on the blocks' half of the packed scan.
-struct WriteBlockScan {
-    WriteScanAndBlocks w;
-    __device__ void operator()(int64_t j, int64_t incl, int64_t item) const {
-        w(j, incl & kLow32, (int32_t)(item & kLow32));
+        return (((r.z - 1) >> sx) - ((r.x - 1) >> sx) + 1) * (((r.w - 1) >> sy) - ((r.y - 1) >> sy) + 1);
     }
 };
 
@@ -1295,8 +1284,11 @@ static bool direct_lists(int64_t n, const BinGeom& g, int64_t key_cap) {
            ceil_div(n, nt) * g.nblocks() * g.tpb() <= 4 * key_cap;
 }
 
-// One workgroup: dc[kCntCoarse] = the sum of the presort's packed counts ((M << 32) | coarse entries),
-// with device counts the frame's status (as k_emit_count), and zero[0, nzero) cleared.
+// One workgroup: dc[1] = M and dc[kCntCoarse] = the coarse entries from the sum of the presort's packed
+// counts (which cannot overflow: direct_lists takes at most kDirectTests Gaussians x blocks, of at most
+// 256 tiles, so M stays below 2^31), with device counts the frame's status (as k_emit_count), and
+// zero[0, nzero) cleared.
+static_assert(kDirectTests * 256 < 2147483648.0, "M of a direct frame");
 __global__ __launch_bounds__(1024) void k_direct_counts(const int64_t* __restrict__ sums, int64_t nsums, int64_t* dc,
                                                         int device_counts, int64_t key_cap, int32_t* zero,
                                                         int64_t nzero) {
@@ -1311,11 +1303,11 @@ __global__ __launch_bounds__(1024) void k_direct_counts(const int64_t* __restric
     if (t != 0) return;
     int64_t packed = 0;
     for (int k = 0; k < 1024 / kWave; ++k) packed += s_w[k];
-    dc[kCntCoarse] = packed;
-    if (!device_counts) return;
     const int64_t keys = packed >> 32;
-    const int64_t st = keys > key_cap ? kFrameKeyCapacity : keys >= (int64_t)INT32_MAX ? kFrameKeyRange : kFrameOk;
     dc[1] = keys;
+    dc[kCntCoarse] = packed & kLow32;
+    if (!device_counts) return;
+    const int64_t st = keys > key_cap ? kFrameKeyCapacity : keys >= (int64_t)INT32_MAX ? kFrameKeyRange : kFrameOk;
     dc[kCntKeysUsed] = st == kFrameOk ? keys : 0;
     dc[kCntCoarseUsed] = st == kFrameOk ? (packed & kLow32) : 0;
     dc[kCntStatus] = st;
@@ -2648,9 +2640,9 @@ int tdgs_render(tdgs_ctx* ctx, void* stream, const tdgs_gaussians* g, const tdgs
             TDGS_LAUNCHED();
         } else {
             StageScope sc(TDGS_STAGE_COUNT_SCAN, s);
-            const SortedTileBlockCounts stb{r.srect, bg.sx, bg.sy, d_nb};
-            TDGS_TRY(device_scan_apply(stb, WriteBlockScan{WriteScanAndBlocks{cs, blk_first, nblk}}, n, r.scan_sums,
-                                       ctx->d_counters + kCntCoarse, s, d_nb));
+            TDGS_TRY(device_scan_apply_packed(SortedBlockCounts{r.srect, bg.sx, bg.sy, d_nb},
+                                              WriteScanAndBlocks{cs, blk_first, nblk}, n, r.scan_sums,
+                                              ctx->d_counters + kCntCoarse, d_m, s, d_nb));
         }
         if (device_counts) {
             // 6-8 sized by the key capacity; the blend copies the counts to the frame counts
@@ -2663,9 +2655,9 @@ int tdgs_render(tdgs_ctx* ctx, void* stream, const tdgs_gaussians* g, const tdgs
         }
         TDGS_TRY(read_counters(ctx, s));
         const int64_t nbf = ctx->h_counters[0];
-        const int64_t m = ctx->h_counters[kCntCoarse] >> 32;
+        const int64_t m = ctx->h_counters[1];
         const int64_t nb = ctx->h_counters[4];
-        const int64_t mc = ctx->h_counters[kCntCoarse] & kLow32;
+        const int64_t mc = ctx->h_counters[kCntCoarse];
         *nb_fgaussians_out = (int32_t)nbf;
         *nb_keys_out = m;
         if (nbf == 0 || m == 0) return launch_render_void(s, cam, opt, out);

@@ -1,7 +1,7 @@
-// scan.hpp — device-wide inclusive scan of int32 (or int64) items with int64 running sums
+// scan.hpp — device-wide inclusive scan of int32 items with int64 running sums
 // (replaces CUDA.jl's accumulate!(+) at src/forward_core.jl:231, 259 and
 // src/training.jl:384). Reduce-then-scan in two launches (or the second alone when the
-// producer of the items sums the tiles, device_scan_apply):
+// producer of the items sums the tiles, device_scan_apply_packed):
 //   1. each 2048-item tile reduces its items                      (k_scan_reduce)
 //   2. each tile sums the earlier tiles' sums into its offset and
 //      rescans its items; tile 0 also writes the total              (k_scan_apply)
@@ -15,6 +15,7 @@
 
 namespace tdgs {
 
+constexpr int64_t kLow32 = 0xffffffffll;
 constexpr int kScanThreads = 256;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kScanThreads * kScanItems;
@@ -65,27 +66,36 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_reduce(In in, int64_t n, 
 }
 
 // Tile b's offset is the sum of tile_sums[0, b); tile 0 sums all ntiles and writes the
-// total to *total_out (when not null).
-template <class In, class Out>
+// total to *total_out (when not null). PACKED: a tile sum holds two counts, the scanned one in its
+// low 32 bits and another above; each is added up in 64 bits of its own (the packed sum of a whole frame's
+// tiles and blocks would overflow), and tile 0 writes the other's total to *total_high.
+template <bool PACKED, class In, class Out>
 __global__ __launch_bounds__(kScanThreads) void k_scan_apply(In in, Out out, int64_t n, const int64_t* tile_sums,
-                                                             int64_t ntiles, int64_t* total_out,
+                                                             int64_t ntiles, int64_t* total_out, int64_t* total_high,
                                                              const int64_t* d_limit) {
     const int64_t b = blockIdx.x;
     const bool past = d_limit && b * kScanTile >= *d_limit;
     if (past && b != 0) return;
     const int64_t upto = b == 0 ? ntiles : b;
-    int64_t part = 0;
-    for (int64_t k = threadIdx.x; k < upto; k += kScanThreads) part += tile_sums[k];
+    int64_t part = 0, high = 0;
+    for (int64_t k = threadIdx.x; k < upto; k += kScanThreads) {
+        const int64_t s = tile_sums[k];
+        part += PACKED ? s & kLow32 : s;
+        if (PACKED) high += s >> 32;
+    }
     int64_t before;
     block_exclusive_scan(part, &before);   // (only the block total is used)
     if (b == 0) {
         if (threadIdx.x == 0 && total_out) *total_out = before;
+        if (PACKED) {
+            block_exclusive_scan(high, &before);
+            if (threadIdx.x == 0) *total_high = before;
+        }
         before = 0;
     }
     if (past) return;
     const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
-    using Item = decltype(in(int64_t(0)));   // int32_t, or int64_t for two packed counts
-    Item v[kScanItems];
+    int32_t v[kScanItems];
     int64_t acc = 0;
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) {
@@ -122,19 +132,20 @@ int device_scan(In1 in_reduce, In2 in_apply, Out out, int64_t n, void* temp, siz
     int64_t* tile_sums = (int64_t*)temp;
     k_scan_reduce<<<(unsigned)ntiles, kScanThreads, 0, stream>>>(in_reduce, n, tile_sums, d_limit);
     TDGS_LAUNCHED();
-    k_scan_apply<<<(unsigned)ntiles, kScanThreads, 0, stream>>>(in_apply, out, n, tile_sums, ntiles, d_total,
-                                                                 d_limit);
+    k_scan_apply<false><<<(unsigned)ntiles, kScanThreads, 0, stream>>>(in_apply, out, n, tile_sums, ntiles, d_total,
+                                                                       nullptr, d_limit);
     TDGS_LAUNCHED();
     return TDGS_OK;
 }
 
 // The apply pass alone, for a producer that has already summed the items of every kScanTile
-// tile into tile_sums (ceil(n / kScanTile) entries).
+// tile into tile_sums (ceil(n / kScanTile) entries) with another count above them (PACKED).
 template <class In, class Out>
-int device_scan_apply(In in, Out out, int64_t n, const int64_t* tile_sums, int64_t* d_total, hipStream_t stream,
-                      const int64_t* d_limit = nullptr) {
+int device_scan_apply_packed(In in, Out out, int64_t n, const int64_t* tile_sums, int64_t* d_total, int64_t* d_high,
+                             hipStream_t stream, const int64_t* d_limit = nullptr) {
     const int64_t ntiles = ceil_div(n > 0 ? n : 1, kScanTile);
-    k_scan_apply<<<(unsigned)ntiles, kScanThreads, 0, stream>>>(in, out, n, tile_sums, ntiles, d_total, d_limit);
+    k_scan_apply<true><<<(unsigned)ntiles, kScanThreads, 0, stream>>>(in, out, n, tile_sums, ntiles, d_total, d_high,
+                                                                      d_limit);
     TDGS_LAUNCHED();
     return TDGS_OK;
 }
