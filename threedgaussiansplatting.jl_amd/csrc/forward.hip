@@ -1657,12 +1657,13 @@ __device__ __forceinline__ void blend_batch(uint32_t lds_addr, int32_t idx0, int
 // (the bound check above runs under whatever exec the last step left; v39 is then advanced for
 // every lane that reads: PX = 1 keeps exec = act0, whose lanes are the only ones that read on)
 #define TDGS_OUT(P, I)                                                                                   \
-    [act##P] "+s"(act[I]), [T##P] "+v"(px[I].T), [R##P] "+v"(px[I].C0), [G##P] "+v"(px[I].C1),            \
-        [B##P] "+v"(px[I].C2)
-// (depth and last index are operands only where they are outputs)
-#define TDGS_OUT_D(P, I) , [D##P] "+v"(px[I].D)
-#define TDGS_OUT_L(P, I) , [L##P] "+v"(px[I].last)
-#define TDGS_OUT_DL(P, I) , [D##P] "+v"(px[I].D), [L##P] "+v"(px[I].last)
+    [act##P] "+&s"(act[I]), [T##P] "+&v"(px[I].T), [R##P] "+&v"(px[I].C0), [G##P] "+&v"(px[I].C1),            \
+        [B##P] "+&v"(px[I].C2)
+// (every operand that is written is early-clobbered, the inputs being read until the last step; depth
+// and last index are operands only where they are outputs)
+#define TDGS_OUT_D(P, I) , [D##P] "+&v"(px[I].D)
+#define TDGS_OUT_L(P, I) , [L##P] "+&v"(px[I].last)
+#define TDGS_OUT_DL(P, I) , [D##P] "+&v"(px[I].D), [L##P] "+&v"(px[I].last)
 #define TDGS_OUT_NONE(P, I)
 #define TDGS_IN(P, I)                                                                                    \
     [uu##P] "v"(px[I].uu), [vv##P] "v"(px[I].vv), [uv##P] "v"(px[I].uv), [cu##P] "v"(px[I].cu), [cv##P] "v"(px[I].cv)
