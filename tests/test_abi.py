@@ -118,3 +118,16 @@ def test_new_entry_points_validate_without_gpu(lib):
     cam40 = abi.Camera(width=40, height=40)
     rc = lib.tdgs_render_tiles(None, C.byref(cam40), C.byref(big), C.byref(opts), C.byref(buf), C.byref(out))
     assert rc == abi.TDGS_ERR_INVALID and b"1024" in lib.tdgs_last_error()
+
+
+def test_render_scratch_holds_no_group_sums_past_the_grouped_sorts(lib):
+    """The depth sorts' group sums (cleared every frame) are sized by the slots the grouped sorts take (2.1M),
+    not by the capacity: past that a slot takes 1/8 byte less (4 passes x 256 words per 32768 slots)."""
+    lib.tdgs_render_temp_bytes.restype = C.c_size_t
+    lib.tdgs_render_temp_bytes.argtypes = [C.c_int32, C.c_int64, C.c_void_p]
+    unit = 32768
+
+    def growth(lo, hi):
+        return (lib.tdgs_render_temp_bytes(hi * unit, 1 << 24, None) - lib.tdgs_render_temp_bytes(lo * unit, 1 << 24, None)) / (hi - lo)
+
+    assert abs(growth(8, 64) - growth(64, 256) - 4096) < 64

@@ -540,16 +540,17 @@ struct DsScratch {
     int32_t* aval;
 };
 
-// Whether the bucketed presort handles n slots with the grouped count tables (zgrp_words
-// zeroed words of group sums).
 // Slots up to which the bucket presort is used. Its buckets grow with n (one workgroup each,
 // 256 of them) and the radix passes take over above: measured 55 vs 68 us at 1M slots (1920 x
 // 1080), 200 vs 142 us at 3M (3840 x 2160); the two lines cross near 1.4M.
 constexpr int64_t kDsMaxSlots = 1400000;
+static_assert(kDsMaxSlots <= kRsMaxGroupedTiles * DsTile::kTile, "the bucket pass has grouped count tables");
+// Words of group sums the bucket pass needs for n slots.
+inline int64_t ds_group_words(int64_t n) { return rs_groups(ceil_div(n > 0 ? n : 1, DsTile::kTile)) * kRsBins; }
+// Whether the bucketed presort handles n slots with the grouped count tables (zgrp_words
+// zeroed words of group sums).
 inline bool ds_applicable(int64_t n, int64_t zgrp_words) {
-    const int64_t tiles = ceil_div(n > 0 ? n : 1, DsTile::kTile);
-    return n > 0 && n <= kDsMaxSlots && tiles <= kRsMaxGroupedTiles &&
-           zgrp_words >= rs_groups(tiles) * kRsBins;
+    return n > 0 && n <= kDsMaxSlots && zgrp_words >= ds_group_words(n);
 }
 
 // The presort of n slots of depth keys (fgidx = slot + 1): sorted_f[0..N_b) and the gather;

@@ -2038,10 +2038,15 @@ static int64_t scan_items(int64_t cap, const tdgs_tiling* t) {
     return cap > nt ? cap : nt;
 }
 // The frame's zeroed scratch (cleared by k_keep_counts): the depth sort's group sums (when
-// grouped), the emission pass's group sums (when grouped: decided by the key capacity) and
-// the count scan's tile sums (int64, accumulated by the depth sort's last pass).
+// grouped: decided by the capacity; of as many slots as the grouped sorts take), the emission pass's
+// group sums (when grouped: decided by the key capacity) and the count scan's tile sums (int64,
+// accumulated by the depth sort's last pass).
 static int64_t depth_group_words(int64_t cap) {
-    return radix_tiles<uint32_t>(cap) <= kRsMaxGroupedTiles ? radix_group_words<uint32_t>(cap, 0, 32) : 0;
+    if (radix_tiles<uint32_t>(cap) > kRsMaxGroupedTiles) return 0;
+    const int64_t most = RsTile<uint32_t>::kGroupedTiles * RsTile<uint32_t>::kTile;
+    const int64_t buckets = ds_group_words(cap < kDsMaxSlots ? cap : kDsMaxSlots);
+    const int64_t radix = radix_group_words<uint32_t>(cap < most ? cap : most, 0, 32);
+    return buckets > radix ? buckets : radix;
 }
 static int64_t emit_group_words(int64_t key_cap) {
     const int64_t tiles = radix_tiles<uint16_t>(key_cap);
