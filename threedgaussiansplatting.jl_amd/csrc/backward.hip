@@ -15,6 +15,7 @@
 // wavefront in LDS, added over the workgroup's wavefronts, and reach global memory once per
 // (tile, Gaussian) — 9 atomics per tile instead of 9 per pixel.
 #include "internal.hpp"
+#include "blend_cuts.hpp"
 #include "wave_sum.hpp"
 
 namespace tdgs {
@@ -79,23 +80,6 @@ struct __align__(16) BackRec {
     float4 c;  // g b f M11     (f: the Gaussian's index, for the flush)
     float4 d;  // M21 M22 r_x r_y
 };
-
-// The half sides (r_x, r_y) of a box around the mean outside which x < cut, for x = -(p du^2 + q du dv +
-// s dv^2) with p, s > 0: x = cut is an ellipse whose du reaches sqrt(-cut s / (p s - q^2 / 4)). The
-// determinant in double (p s and q^2 / 4 agree to 1 in 1e4 and more for needles), the box widened by
-// 1e-4 of its size and 1e-2 pixels for the rounding of x, the cut and the square root; no bound
-// (infinite sides) where the form is not definite or anything is NaN, none at all (negative
-// sides) where a positive cut says that no alpha reaches min_alpha. The cut's own margin (1e-3) covers its error.
-__device__ __forceinline__ void cut_box(float A, float B, float C, float cut, float* rx, float* ry) {
-    const float p = -A, s = -C;
-    const double det = (double)p * s - 0.25 * (double)B * B;
-    const float k = -cut / (float)det;
-    const float x2 = k * s, y2 = k * p;
-    const bool bounded = p > 0.0f && s > 0.0f && det > 0.0 && x2 >= 0.0f && y2 >= 0.0f && x2 < kInf && y2 < kInf;
-    *rx = bounded ? fmaf(sqrtf(x2), 1.0001f, 0.01f) : kInf;
-    *ry = bounded ? fmaf(sqrtf(y2), 1.0001f, 0.01f) : kInf;
-    if (cut > 1e-3f) *rx = *ry = -kInf;
-}
 
 struct BackBlendArgs {
     int32_t W, H, TW, TH, ntx;

@@ -37,6 +37,7 @@
 
 #include "dsort.hpp"
 #include "internal.hpp"
+#include "blend_cuts.hpp"
 #include "scan.hpp"
 #include "sort.hpp"
 

@@ -53,38 +53,6 @@ struct StageScope {
     ~StageScope() { profile_mark(stage, false, stream); }
 };
 
-// Exponent below which blending can skip an entry: for e < exponent_cut(min_alpha),
-// exp_f(e) (relative error a few 1e-7) is below min_alpha, so alpha < min_alpha. A margin of
-// 1e-3 in the exponent covers the rounding; no cut without a positive min_alpha.
-inline float exponent_cut(float min_alpha) {
-    if (!(min_alpha > 0.0f)) return -__builtin_inff();
-    return std::nextafter((float)(std::log((double)min_alpha) - 1e-3), -__builtin_inff());
-}
-
-// The exponent from which alpha = exp_f(e) reaches min_alpha: exp_f(e) >= min_alpha exactly for e >= *cut.
-// exp_f is within 0.91 ulp (1.1e-7 relative) of a strictly rising function and neighbouring exponents of
-// at least 1 in size lie 1.2e-7 apart or more, so there the switch is at most two floats from
-// log(min_alpha) rounded and is looked for within four; within 32 up to a min_alpha of 0.9, where
-// the exponents lie at least 7e-9 apart. It has to be a clean one. (Each look costs the host ~40 ns, which a
-// frame with host counts waits for.) False when there is none, when max_alpha stays below min_alpha,
-// or when *cut < -80 (results of exp_f near its flush to zero).
-inline bool exact_exponent_cut(float min_alpha, float max_alpha, float* cut) {
-    *cut = 0.0f;
-    if (!(min_alpha > 0.0f) || !(min_alpha <= 0.9f) || !(max_alpha >= min_alpha)) return false;
-    const float mid = (float)std::log((double)min_alpha);   // negative: one float up is one less in the bits
-    if (!(mid >= -80.0f)) return false;
-    const int span = mid <= -1.0f ? 4 : 32;
-    bool reached = false;
-    for (int k = -span; k < span; ++k) {
-        const float e = bits_float(float_bits(mid) - (uint32_t)k);
-        const bool r = exp_f(e) >= min_alpha;
-        if (r ? k == -span : reached) return false;
-        if (r && !reached) *cut = e;
-        reached = r;
-    }
-    return reached;
-}
-
 // Pixel of thread t inside a TW x TH tile (1-based). With both sides multiples of 8 each
 // wavefront covers an 8x8 block (blocks column-major, lanes column-major inside), which
 // keeps a Gaussian's footprint inside as few wavefronts as possible; otherwise wavefront
