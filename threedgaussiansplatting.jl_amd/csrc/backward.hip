@@ -137,8 +137,7 @@ constexpr size_t kBackLds = 56 << 10; // LDS of a workgroup, at most
 // What bounds the filled chip is VALU issue: ~75 instructions an entry (x of the four slots, compares,
 // 1.3 live slots' steps, a seventh of a transpose-sum), of which a multiply, add, FMA or move takes 2
 // cycles of a SIMD, a compare, select, DPP, integer or scalar-operand instruction about 4, exp2 and
-// reciprocal 8. Hence one compare per slot for the cut, the one for the last contributor only where
-// the cut leaves the slot, and the transpose-sum by masked DPP adds: 329.6 -> 324.1 us at 1M Gaussians, 1080p, 694 -> 688 us at 3M, 4K.
+// reciprocal 8. Hence the transpose-sum by masked DPP adds: 328 -> 307 us at 1M Gaussians, 1080p.
 template <bool SEP, int PX, int BPC, bool CULL>
 __global__ __launch_bounds__(1024 / PX) __attribute__((amdgpu_waves_per_eu(4))) void k_backward_blend(
     BackBlendArgs a) {
@@ -370,11 +369,11 @@ __global__ __launch_bounds__(1024 / PX) __attribute__((amdgpu_waves_per_eu(4))) 
                             x[p] = fmaf(fmaf(ra.z, du[p], ra.w * dv[p]), du[p], rb.x * dv[p] * dv[p]);
                             live[p] = __builtin_amdgcn_ballot_w64(!(x[p] < rb.y));
                         }
-                        // A compare costs the issue slots of two multiply-adds: the pixels' last
-                        // contributors are looked at only for the slots the entry reaches.
+                        // (both compares of every slot, without branches: the last contributor's only for the
+                        // slots the cut leaves, behind a branch each, took 319 us against 307 at 1M Gaussians, 1080p)
 #pragma unroll
                         for (int p = 0; p < PX; ++p) {
-                            if (live[p] != 0) live[p] &= __builtin_amdgcn_ballot_w64(jj < last_rel[p]);
+                            live[p] &= __builtin_amdgcn_ballot_w64(jj < last_rel[p]);
                             any |= live[p];
                         }
                         if (any == 0) continue;
