@@ -218,3 +218,25 @@ def test_backward_no_alpha_in_range(gpu):
     fg = gpu.FilteredGaussiansGradientsVector(buf.capacity, 0, 0)
     gpu.backward_(fg, torch.ones_like(out.rgb), out, g, cam, t, opts, buf)
     assert buf.nb_keys > 0 and float(fg.grads2d.abs().max()) == 0.0 and int(out.last.max()) == 0
+
+
+@pytest.mark.parametrize("w,h,tile", [(330, 250, (24, 24)), (655, 636, (24, 24)), (720, 720, (24, 24)),
+                                      (655, 636, (20, 20)), (655, 636, (48, 16)), (655, 636, (4, 100))])
+@pytest.mark.parametrize("scene", ["usual", "needles"])
+def test_backward_slots_of_no_constant_offset(gpu, oracle, w, h, tile, scene):
+    """Tiles whose slots have boxes of their own: three 8 x 8 blocks per column (9 blocks, an odd slot
+    left over), runs of columns, pieces of a column longer than a slot; one, two and four pixels per lane."""
+    g = synthetic.config(0, n=1500).gaussians
+    if scene == "needles":
+        g.scaling[:] = np.random.default_rng(3).uniform(-6.0, 0.0, g.scaling.shape).astype(np.float32)
+    cam = host.look_at_camera(w, h, 60.0, (0.0, 0.0, -4.0))
+    t = host.Tiling.for_camera(cam, *tile)
+    opts = host.RenderOptions.for_camera(cam, 0, background_color=(0.2, 0.1, 0.3))
+    gen = torch.Generator(device="cuda").manual_seed(17)
+
+    def rand_grad(rgb):
+        return (torch.rand(rgb.shape, generator=gen, device=rgb.device) - 0.5) * 1e-3
+
+    got, ref = _run(gpu, oracle, g, cam, t, opts, rand_grad)
+    for k in ["grads2d"] + (ARRAYS if scene == "usual" else []):
+        assert rel_l2(got[k], ref[k]) <= REL_L2, (k, rel_l2(got[k], ref[k]))

@@ -194,12 +194,37 @@ __global__ __launch_bounds__(1024 / PX) __attribute__((amdgpu_waves_per_eu(4))) 
         cv[p] = (float)V - 0.5f;
     }
     static_assert(BPC == 0 || PX % BPC == 0 || BPC % PX == 0, "constant slot offsets");
-    // The box of slot 0's pixel centres: corner (box_u, box_v), an 8 x 8 block, the others' moved as the
-    // slots are; the whole tile for every slot where the slots are no blocks (BPC = 0 but for PX = 1).
-    const bool blocks = BPC != 0 || (PX == 1 && ((a.TW | a.TH) & 7) == 0);
-    const int block0 = blocks ? __builtin_amdgcn_readfirstlane(t / kWave) * PX : 0;   // column-major
-    const int bpc = blocks ? a.TH >> 3 : 1;
-    const int box_u = (tx - 1) * a.TW + 8 * (block0 / bpc), box_v = (ty - 1) * a.TH + 8 * (block0 % bpc);
+    // CULL: the box of a slot's pixel centres, its middle (box_u, box_v) and half sides: an 8 x 8 block of
+    // the tile (column-major), or the columns its 64 pixels lie in where the tile's sides are no multiples of 8
+    // (tile_pixel). With BPC the others' are slot 0's, moved as the slots are. (The whole tile as the box of
+    // every slot without BPC lost more than the culling gave: 60k and 200k Gaussians, 720x720, 20x20 tiles 85 and
+    // 207 us, now 72 and 191, walking every entry 117 and 195; 500k, 608x608 307, 236, 342.)
+    constexpr int kBoxes = BPC == 0 ? PX : 1;
+    float box_u[kBoxes], box_v[kBoxes], half_u[kBoxes], half_v[kBoxes];
+    if (CULL) {
+#pragma unroll
+        for (int p = 0; p < kBoxes; ++p) {
+            const int block = __builtin_amdgcn_readfirstlane(t / kWave) * PX + p;
+            int u_lo, u_hi, v_lo, v_hi;
+            if (BPC != 0 || ((a.TW | a.TH) & 7) == 0) {
+                const int bpc = BPC != 0 ? BPC : a.TH >> 3;
+                u_lo = 8 * (block / bpc);
+                v_lo = 8 * (block % bpc);
+                u_hi = u_lo + 7;
+                v_hi = v_lo + 7;
+            } else {
+                const int i_lo = kWave * block, i_hi = i_lo + kWave - 1 < NT ? i_lo + kWave - 1 : NT - 1;
+                u_lo = i_lo / a.TH;
+                u_hi = i_hi / a.TH;
+                v_lo = u_lo == u_hi ? i_lo % a.TH : 0;
+                v_hi = u_lo == u_hi ? i_hi % a.TH : a.TH - 1;
+            }
+            half_u[p] = 0.5f * (float)(u_hi - u_lo);
+            half_v[p] = 0.5f * (float)(v_hi - v_lo);
+            box_u[p] = (float)((tx - 1) * a.TW + u_lo) + 0.5f + half_u[p];
+            box_v[p] = (float)((ty - 1) * a.TH + v_lo) + 0.5f + half_v[p];
+        }
+    }
     const int slot = lane / 9, comp = lane - 9 * slot;
     const int partner = comp == 0 ? lane + 1 : comp == 1 ? lane - 1 : lane;
     const float scale = comp == 4 ? -1.0f : (comp == 3 || comp == 5) ? -0.5f : 1.0f;
@@ -290,13 +315,12 @@ __global__ __launch_bounds__(1024 / PX) __attribute__((amdgpu_waves_per_eu(4))) 
                 mx = m.x; my = m.y; rx = r.x; ry = r.y;
             }
             cand_any = 0;
-            const float hu = blocks ? 3.5f : 0.5f * (float)a.TW, hv = blocks ? 3.5f : 0.5f * (float)a.TH;
-            const float ou = mx - ((float)box_u + 0.5f + hu), ov = my - ((float)box_v + 0.5f + hv);
-            const float wu = rx + hu, wv = ry + hv;
 #pragma unroll
             for (int p = 0; p < PX; ++p) {
-                const bool hit = !(fabsf(ou - (float)(BPC ? 8 * (p / (BPC ? BPC : 1)) : 0)) > wu) &&
-                                 !(fabsf(ov - (float)(BPC ? 8 * (p % (BPC ? BPC : 1)) : 0)) > wv);
+                const int q = BPC == 0 ? p : 0;
+                const float ou = mx - box_u[q] - (float)(BPC ? 8 * (p / (BPC ? BPC : 1)) : 0);
+                const float ov = my - box_v[q] - (float)(BPC ? 8 * (p % (BPC ? BPC : 1)) : 0);
+                const bool hit = !(fabsf(ou) > rx + half_u[q]) && !(fabsf(ov) > ry + half_v[q]);
                 cand[p] = __builtin_amdgcn_ballot_w64(hit);
                 cand_any |= cand[p];
             }
