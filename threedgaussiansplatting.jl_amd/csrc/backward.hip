@@ -110,25 +110,39 @@ struct BackBlendArgs {
 // fewer entries reach: with CULL a batch's entries are first tested, one per lane, by their boxes
 // against each slot's block, and the walk visits only those that reach it. The work grows (the
 // sums over the wavefront serve fewer pixels), so the filled chip keeps four pixels per lane, where
-// CULL's branches per slot cost more than the dead slots they skip (368 against 314 us at the
-// last line below). us, by 64-pixel blocks of the image, and image, Gaussians, tiles:
-//                                             PX = 4       2       1   (always 4 and every entry walked)
-//     520   200x150     3k  16x16               76.2    45.3    28.5   (76.4)
-//    1024   256x256    10k  16x16              178.3   105.7    63.4   (177.9)
-//    2500   400x400    20k  16x16              213.7   133.5    84.5   (211.8)
-//    4800   640x480   500k  16x16              298.4   203.4   177.8   (289.6)
-//    5776   600x600    60k  16x16              179.7   128.0   112.4   (174.8)
-//    8928   979x546    60k  16x32               93.9    59.2    64.3   (91.5)
-//   10000   800x800   200k  16x16              161.1   171.9   171.2   (162.3)
-//   17384   1297x840  500k  16x16              252.6   265.6   295.8   (259.3)
-//   32640   1920x1080   1M  16x16              324.1   371.7   440.8   (329.6)
-// Tiles of at most 64 PX / 2 pixels would leave half the lanes off (8 x 8 tiles, 800x600, 200k:
-// 180.6, 165.5, 143.2).
+// CULL's branches per slot cost more than the dead slots they skip (368 against 314 us at 1M
+// Gaussians, 1080p). us of the three, one scene at sizes on both sides of the lines, by 64-pixel blocks:
+// R 60k small Gaussians in a room, B 200k of one object, D 100k large ones.
+//                             R: PX = 4     2     1   B: PX = 4     2     1   D: PX = 4     2     1
+//     2500   400x400  16x16      151.0  93.2  60.2     197.5 148.6  94.8     125.0 103.7  71.6
+//     5776   608x608  16x16      101.1  69.8  48.0     161.5 139.6 131.4     115.5 112.3 108.2
+//     6384   660x600  16x16      100.4  66.4  52.9     155.7 132.7 132.6     125.0 109.7 110.2
+//     8100   720x720  16x16       90.6  64.4  55.0     160.0 136.2 148.4     120.8 112.1 124.4
+//     8928   979x546  16x32       91.9  61.2  67.9     155.7 142.6 153.5     125.3 126.6 141.6
+//    10000   800x800  16x16       84.7  62.7  58.6     164.2 171.8 169.4     131.0 152.5 154.3
+//    12288  1024x768  16x16       75.3  70.0  70.7     165.1 170.4 181.0     130.7 153.7 168.2
+//    14400  1280x720  16x16       68.7  71.2  79.0     162.2 176.7 195.6     136.1 169.3 183.5
+// Short lists gain from few pixels per lane past both lines, long ones lose. A launch knows the image and not the
+// lists (their length stays on the device), so the lines lie where the long lists' loss is still small (D to 5%) beside the
+// short ones' gain: 1.5 rounds of the resident wavefronts with one pixel per lane, 1.125 with two.
+// Workgroups of more than four wavefronts: a CU holds as many as its fullest SIMD takes (two of five, one of
+// nine), so they also must fit back_fits' rounds. 24x24 tiles at PX = 4, 2, 1: 720x720 (900 tiles, 512 of five
+// wavefronts at a time) 111.5, 86.7, 98.6 (R), 183.5, 234.2, 243.1 (B), 136.8, 186.1, 200.3 (D); 660x600 (700
+// tiles) 127.7, 76.6, 74.4; 186.1, 186.8, 201.2; 132.2, 139.6, 162.1.
+// Tiles of at most 64 PX / 2 pixels would leave half the lanes off (8 x 8 tiles, 800x800: 67.8, 65.0, 58.3; 210.3,
+// 201.7, 178.4; 257.7, 268.0, 250.8).
 constexpr int64_t kBackWaves1 = 6144, kBackWaves2 = 9216;   // blocks up to which PX is 1, 2
+constexpr int kCUs = 256;
+// Whether the tiles' workgroups of px pixels per lane take at most two (px = 1) or one and a half (2) rounds of the
+// chip. Up to four wavefronts fill a CU evenly, and the lines above decide.
+static bool back_fits(int64_t tiles, int pixels, int px) {
+    const int64_t nw = ceil_div(pixels, px * kWave);
+    return nw <= 4 || 2 * tiles <= (px == 1 ? 4 : 3) * kCUs * (4 / ceil_div(nw, 4));
+}
 constexpr int kBackBatch = 128;       // entries per batch with PX < 4, at most (64: 5% slower; 256: the same)
 constexpr size_t kBackLds = 56 << 10; // LDS of a workgroup, at most
 // BPC > 0 (tile sides multiples of 8, BPC = TH / 8 blocks of 8 x 8 pixels per block column,
-// BPC dividing PX): slot p's pixels are slot 0's moved by the constant (8 (p / BPC), 8 (p %
+// BPC dividing PX or PX dividing BPC): slot p's pixels are slot 0's moved by the constant (8 (p / BPC), 8 (p %
 // BPC)), so only slot 0's coordinates are kept per lane and the others' offsets from the
 // record are slot 0's plus a constant (three fewer register pairs: 323 us against 349 us at 1M
 // Gaussians, 1080p, where the loop's scratch spills went from 52 to 12 bytes per lane). The
@@ -145,7 +159,7 @@ __global__ __launch_bounds__(1024 / PX) __attribute__((amdgpu_waves_per_eu(4))) 
     const int NT = a.TW * a.TH;
     const int NTH = (int)blockDim.x, NB = a.batch;
     BackRec* s_rec = reinterpret_cast<BackRec*>(s_raw4);
-    // Per-wavefront sums [wave][NB][9] (at most 4 wavefronts: 1024 / PX threads). A wavefront
+    // Per-wavefront sums [wave][NB][9] (at most 16 / PX wavefronts: 1024 / PX threads). A wavefront
     // takes each entry into at most one slot, so its transposed sums are plain stores (an LDS
     // atomic's round trip sat in front of the next entry's record reads); the flush adds the
     // wavefronts' copies.
@@ -893,8 +907,10 @@ int tdgs_backward_render_tiles(void* stream, tdgs_gradients* grads, const float*
     // px pixels per thread, in whole wavefronts (the transpose-sum reads all 64 lanes; the pixels
     // past the tile's are off); see k_backward_blend for the choice.
     const int pixels = tiling->tile_width * tiling->tile_height;
-    const int64_t blocks = (int64_t)tiling->nb_tiles_x * tiling->nb_tiles_y * ceil_div(pixels, kWave);
-    const int px = pixels <= kWave || blocks <= kBackWaves1 ? 1 : pixels <= 2 * kWave || blocks <= kBackWaves2 ? 2 : 4;
+    const int64_t tiles = (int64_t)tiling->nb_tiles_x * tiling->nb_tiles_y, blocks = tiles * ceil_div(pixels, kWave);
+    const int px = pixels <= kWave || (blocks <= kBackWaves1 && back_fits(tiles, pixels, 1))       ? 1
+                   : pixels <= 2 * kWave || (blocks <= kBackWaves2 && back_fits(tiles, pixels, 2)) ? 2
+                                                                                                   : 4;
     const int nt = (int)ceil_div(pixels, px * kWave) * kWave;
     const int nw = nt / kWave;
     a.batch = px == 4 || nt < kBackBatch ? nt : kBackBatch;
