@@ -392,3 +392,26 @@ def test_render_extreme_covariances_bit_exact(gpu, oracle, w, h, dilation):
     np.testing.assert_array_equal(out.rgb.cpu().numpy(), r["rgb"])
     np.testing.assert_array_equal(out.T.cpu().numpy(), r["T"])
     np.testing.assert_array_equal(out.last.cpu().numpy(), r["last"])
+
+
+@pytest.mark.parametrize("min_alpha,max_alpha", [(1 / 255, 0.99), (0.92, 0.99), (0.5, 0.3), (1.7e-38, 0.99), (0.01, 1e38)])
+@pytest.mark.parametrize("w,h", [(256, 256), (2048, 1600)])
+def test_render_exponents_of_any_size_bit_exact(gpu, oracle, min_alpha, max_alpha, w, h):
+    """Batches that hold records of exponents far above 88 (opacities to 3e38 and infinite), next to usual ones,
+    for thresholds with and without an exponent that stands for min_alpha; one and two pixels per lane."""
+    from tdgs_amd import ply
+    wl = synthetic.config(0, n=1200)
+    ro = ply.to_render_only(wl.gaussians)
+    ro.means_opacity[::97, 3] = np.float32(3e38)
+    ro.means_opacity[5::197, 3] = np.float32(np.inf)
+    ro.means_opacity[11::89, 3] = np.float32(2e9)
+    ro.means_opacity[:200, 3] = np.linspace(0.0, 4.0, 200, dtype=np.float32)
+    cam = host.look_at_camera(w, h, 60.0, (0.0, 0.0, -4.0))
+    t = host.Tiling.for_camera(cam, 16, 16)
+    opts = host.RenderOptions.for_camera(cam, 0, min_alpha=min_alpha, max_alpha=max_alpha)
+    r = oracle.render(ro, cam, t, opts)
+    g = gpu.RenderOnlyGaussiansVector.from_host(ro, 0)
+    out = gpu.RenderOutputs.for_camera(cam, 0, include_depth=True)
+    gpu.render_(out, g, cam, t, opts, gpu.RenderBuffers(len(g), t, 0))
+    for name in ("rgb", "T", "depth", "last"):
+        np.testing.assert_array_equal(getattr(out, name).cpu().numpy(), r[name])

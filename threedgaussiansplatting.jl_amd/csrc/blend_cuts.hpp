@@ -16,15 +16,16 @@ inline float exponent_cut(float min_alpha) {
     return std::nextafter((float)(std::log((double)min_alpha) - 1e-3), -__builtin_inff());
 }
 
-// The exponent from which alpha = exp_f(e) reaches min_alpha: exp_f(e) >= min_alpha exactly for e >= *cut.
-// exp_f is within 0.91 ulp (1.1e-7 relative) of a strictly rising function and neighbouring exponents of
-// at least 1 in size lie 1.2e-7 apart or more, so there the switch is at most two floats from
-// log(min_alpha) rounded and is looked for within four; within 32 up to a min_alpha of 0.9, where
-// the exponents lie at least 7e-9 apart. It has to be a clean one. (Each look costs the host ~40 ns, which a
-// frame with host counts waits for.) False when there is none, when max_alpha stays below min_alpha,
-// or when *cut < -80 (results of exp_f near its flush to zero).
+// The exponent from which alpha = min(exp_f(e), max_alpha) reaches min_alpha: alpha >= min_alpha exactly for
+// e >= *cut (infinity where max_alpha stays below min_alpha). exp_f is within 0.91 ulp (1.1e-7 relative) of exp, so only
+// exponents within 1.1e-7 of log(min_alpha) are in doubt: two floats to either side where the exponents are at least 1
+// in size (1.2e-7 apart or more), looked for within four; 15 up to a min_alpha of 0.9 (7.4e-9 apart), looked for within
+// 32. The switch among them has to be a clean one (above a min_alpha of 1/e several neighbouring exponents share
+// an alpha, and exp_f may step back by an ulp). (Each look costs the host ~40 ns, which a frame with host counts waits for.) False when there is
+// none, or when *cut < -80 (results of exp_f near its flush to zero).
 inline bool exact_exponent_cut(float min_alpha, float max_alpha, float* cut) {
-    *cut = 0.0f;
+    *cut = __builtin_inff();
+    if (max_alpha < min_alpha) return true;
     if (!(min_alpha > 0.0f) || !(min_alpha <= 0.9f) || !(max_alpha >= min_alpha)) return false;
     const float mid = (float)std::log((double)min_alpha);   // negative: one float up is one less in the bits
     if (!(mid >= -80.0f)) return false;

@@ -1491,7 +1491,7 @@ struct BlendArgs {
     float e_cut;     // exp_f(e) < min_alpha for every exponent e < e_cut (with a margin)
     float e_exact;   // exp_f(e) >= min_alpha exactly for the exponents e >= e_exact
     int32_t batch;   // records per batch, at most the tile's pixels
-    int checked;     // no such e_exact, or below exp_f's polynomial range: batches take the compiled loop
+    int32_t steps;   // kSteps* of its batches
     int64_t m;
     const int32_t* tiles_end;
     const int32_t* sorted_f;
@@ -1510,18 +1510,25 @@ struct BlendArgs {
     int64_t* mon_host;
 };
 
+// The steps a batch takes: blend_batch with one compare for min_alpha (e_exact); with two compares and exponents
+// of any size, for batches that hold an odd record or thresholds without an e_exact; the compiled loop, for
+// thresholds outside exp_f's polynomial range.
+enum : int32_t { kStepsExact = 0, kStepsGeneral = 1, kStepsCompiled = 2 };
+
 // The blending steps of one batch of staged records, written out instruction by instruction, for one
 // or two pixels per lane (PX). Per record and pixel it performs exactly the single-precision
 // operations of the C++ loop in k_render_tiles below (same operands, same order: the exponent's
 // five fused multiply-adds, exp_f_core's sequence, min with max_alpha, 1 - alpha, the products and
 // the colour fused multiply-adds), so every result is bit for bit the compiled loop's, in cheaper
 // steps:
-//   - the contributing lanes are those with e >= e_exact, one compare for the loop's two (e_cut,
-//     min_alpha): exp_f rises strictly from one float to the next around min_alpha, so
-//     alpha >= min_alpha says the same as e >= e_exact (exact_exponent_cut);
+//   - EXACT: the contributing lanes are those with e >= cut = e_exact, one compare for the loop's two (e_cut,
+//     min_alpha): the lowest exponent whose alpha reaches min_alpha, all below it falling short and all above
+//     reaching it (exact_exponent_cut looks for it). Otherwise cut = e_cut, alpha is compared with min_alpha as
+//     the loop does, and exponents above 88 or NaN become 88 (v_min with a NaN gives the other operand): exp_f(88) =
+//     1.65e38 is above max_alpha, as are the loop's larger values, and the loop's min of a NaN is max_alpha too;
 //   - n = rint(x log2 e) comes from adding and subtracting 1.5 2^23 (the same ties-to-even rounding),
 //     which leaves n in the sum's low mantissa bits; shifted to the exponent field and added to
-//     exp_poly's bits they are the product with 2^n (exact: the exponents are at least -80, so
+//     exp_poly's bits they are the product with 2^n (exact: the exponents are at least -87, so
 //     nothing is subnormal). A compare, a conversion, a v_rndne, an integer or scalar-operand
 //     instruction takes 4 cycles of a SIMD where an add, multiply or FMA takes 2; a v_ldexp with the
 //     conversion it needs takes 8;
@@ -1530,7 +1537,10 @@ struct BlendArgs {
 // The next record is read from LDS into a second register set while the current one is processed, so
 // no step waits on LDS. Records run in groups of four with one bound check per group: after a
 // batch the LDS array holds three records of padding that no pixel is live for, and one
-// more for the read past the last group. Valid only for batches that are not `checked`.
+// more for the read past the last group. For kStepsExact and kStepsGeneral batches. (Without the general
+// steps such batches took the compiled loop; us with both compares in every batch | the loop | the general steps: 1M
+// Gaussians, 1080p, min_alpha 0.92 21.1 | 24.9 | 22.4; max_alpha below min_alpha 64 | 106 | 57 (an infinite e_exact);
+// 10k needles, 1080p 28.0 | 32.0 | 29.1. The loop starts on an instruction cache line: 415 -> 413 us at 1M, 3840x2160.)
 //
 // PX = 2: an LDS read of a record (three reads, 11 cycles of the CU's LDS pipe, shared by its four
 // SIMDs) and the loop's scalar instructions serve two 8 x 8 blocks of the tile; each block is
@@ -1559,10 +1569,11 @@ struct BlendPx {
 };
 
 // Steps through records idx0 .. idx_end - 1 (1-based sorted indices) staged at lds_addr; act[k] is the
-// mask of the lanes whose pixel k is still blending, on entry and on return. v37-v63 are
-// scratch registers (the kernel stays within 64 VGPRs, 8 wavefronts per SIMD).
-template <bool DEPTH, bool LAST, int PX>
-__device__ __forceinline__ void blend_batch(uint32_t lds_addr, int32_t idx0, int32_t idx_end, float e_exact,
+// mask of the lanes whose pixel k is still blending, on entry and on return. v38-v63 are
+// scratch registers (the kernel stays within 64 VGPRs with one pixel per lane, 8 wavefronts per SIMD, and within
+// 80 with two, 6).
+template <bool EXACT, bool DEPTH, bool LAST, int PX>
+__device__ __forceinline__ void blend_batch(uint32_t lds_addr, int32_t idx0, int32_t idx_end, float cut, float min_alpha,
                                             float max_alpha, float min_T, BlendPx (&px)[PX], uint64_t (&act)[PX]) {
     const float c5 = kExpC5;   // exp_poly's coefficient of r^5 (a VGPR operand)
     uint64_t ent, lv;
@@ -1575,7 +1586,8 @@ __device__ __forceinline__ void blend_batch(uint32_t lds_addr, int32_t idx0, int
     "v_fmac_f32 " E ", " A1 ", %[vv" P "]\n"         \
     "v_fmac_f32 " E ", " A0 ", %[uu" P "]\n"
 // the step of the contributing lanes (exec) of pixel P with exponent E and colour R, G, B
-#define TDGS_LIVE(E, P, ID, K, R, G, B, DEPTH_FMA, LAST_MOV)                                      \
+#define TDGS_LIVE(CLAMP, REACH, E, P, ID, K, R, G, B, DEPTH_FMA, LAST_MOV)                        \
+    CLAMP(E)                                                                                       \
     "v_mul_f32 v61, 0x3fb8aa3b, " E "\n"                                                              \
     "v_add_f32 v61, 0x4b400000, v61\n"                                                                \
     "v_add_f32 v62, 0xcb400000, v61\n"                                                                \
@@ -1588,7 +1600,7 @@ __device__ __forceinline__ void blend_batch(uint32_t lds_addr, int32_t idx0, int
     "v_fma_f32 v63, v63, " E ", 1.0\n"                                                            \
     "v_fma_f32 v63, v63, " E ", 1.0\n"                                                            \
     "v_lshl_add_u32 v63, v61, 23, v63\n"                                                          \
-    "v_min_f32 v63, %[maxa], v63\n"                                                               \
+    "v_min_f32 v63, %[maxa], v63\n" REACH                                                         \
     "v_sub_f32 v61, 1.0, v63\n"                                                                   \
     "v_mul_f32 v61, %[T" P "], v61\n"                                                             \
     "v_cmp_gt_f32 vcc, %[minT], v61\n"                                                            \
@@ -1616,38 +1628,38 @@ __device__ __forceinline__ void blend_batch(uint32_t lds_addr, int32_t idx0, int
     "ds_read_b128 " Q0 ", v39 offset:" O0 "\n"          \
     "ds_read_b128 " Q1 ", v39 offset:" O1 "\n" READ_C(CP, C1, OC)
 // one record: ID = K its number in the group of four, the registers of its set, the next read
-#define TDGS_STEP1(ID, A0, A1, A2, A3, B0, B1, R, G, B, DF, LM, NEXT)                             \
+#define TDGS_STEP1(CL, RE, ID, A0, A1, A2, A3, B0, B1, R, G, B, DF, LM, NEXT)                             \
     "s_waitcnt lgkmcnt(0)\n" NEXT TDGS_EXPONENT("v60", "0", A0, A1, A2, A3, B0, B1)               \
     "v_cmp_ngt_f32 vcc, %[cut], v60\n"                                                            \
     "s_cbranch_vccz .Lsk" ID "0_%=\n"                                                             \
-    "s_mov_b64 exec, vcc\n" TDGS_LIVE("v60", "0", ID, ID, R, G, B, DF("0"), LM("0", ID))          \
+    "s_mov_b64 exec, vcc\n" TDGS_LIVE(CL, RE, "v60", "0", ID, ID, R, G, B, DF("0"), LM("0", ID))          \
     "s_mov_b64 exec, %[act0]\n"                                                                   \
     ".Lsk" ID "0_%=:\n"
-#define TDGS_STEP2(ID, A0, A1, A2, A3, B0, B1, R, G, B, DF, LM, NEXT)                             \
+#define TDGS_STEP2(CL, RE, ID, A0, A1, A2, A3, B0, B1, R, G, B, DF, LM, NEXT)                             \
     "s_waitcnt lgkmcnt(0)\n" NEXT TDGS_EXPONENT("v60", "0", A0, A1, A2, A3, B0, B1)               \
     "v_cmp_ngt_f32 vcc, %[cut], v60\n" TDGS_EXPONENT("v38", "1", A0, A1, A2, A3, B0, B1)          \
     "v_cmp_ngt_f32 %[lv], %[cut], v38\n"                                                          \
     "s_and_b64 exec, vcc, %[act0]\n"                                                              \
-    "s_cbranch_execz .Lsk" ID "0_%=\n" TDGS_LIVE("v60", "0", ID, ID, R, G, B, DF("0"), LM("0", ID))  \
+    "s_cbranch_execz .Lsk" ID "0_%=\n" TDGS_LIVE(CL, RE, "v60", "0", ID, ID, R, G, B, DF("0"), LM("0", ID))  \
     ".Lsk" ID "0_%=:\n"                                                                           \
     "s_and_b64 exec, %[lv], %[act1]\n"                                                            \
-    "s_cbranch_execz .Lsk" ID "1_%=\n" TDGS_LIVE("v38", "1", ID, ID, R, G, B, DF("1"), LM("1", ID))  \
+    "s_cbranch_execz .Lsk" ID "1_%=\n" TDGS_LIVE(CL, RE, "v38", "1", ID, ID, R, G, B, DF("1"), LM("1", ID))  \
     ".Lsk" ID "1_%=:\n"                                                                           \
     "s_mov_b64 exec, %[ent]\n"
 #define TDGS_SET0 "v40", "v41", "v42", "v43", "v44", "v45", "v46", "v47", "v48"
 #define TDGS_SET1 "v50", "v51", "v52", "v53", "v54", "v55", "v56", "v57", "v58"
 #define TDGS_CALL(F, ...) F(__VA_ARGS__)
-#define TDGS_LOOP(STEP, ENTER, RC, DF0, DF1, LM)                                                              \
+#define TDGS_LOOP(STEP, ENTER, CL, RE, RC, DF0, DF1, LM)                                                              \
     "s_mov_b64 %[ent], exec\n"                                                                                \
     "s_mov_b32 %[idx], %[i0]\n"                                                                               \
     "v_mov_b32 v39, %[addr]\n" TDGS_READ(RC, "v[40:43]", "v[44:47]", "v[48:49]", "v48", "0", "16", "32") ENTER \
-    ".Lstep_%=:\n" TDGS_CALL(STEP, "0", TDGS_SET0, DF0, LM,                                                   \
+    ".p2align 6\n.Lstep_%=:\n" TDGS_CALL(STEP, CL, RE, "0", TDGS_SET0, DF0, LM,                                                   \
                              TDGS_READ(RC, "v[50:53]", "v[54:57]", "v[58:59]", "v58", "48", "64", "80"))      \
-        TDGS_CALL(STEP, "1", TDGS_SET1, DF1, LM,                                                              \
+        TDGS_CALL(STEP, CL, RE, "1", TDGS_SET1, DF1, LM,                                                              \
                   TDGS_READ(RC, "v[40:43]", "v[44:47]", "v[48:49]", "v48", "96", "112", "128"))               \
-            TDGS_CALL(STEP, "2", TDGS_SET0, DF0, LM,                                                          \
+            TDGS_CALL(STEP, CL, RE, "2", TDGS_SET0, DF0, LM,                                                          \
                       TDGS_READ(RC, "v[50:53]", "v[54:57]", "v[58:59]", "v58", "144", "160", "176"))          \
-                TDGS_CALL(STEP, "3", TDGS_SET1, DF1, LM,                                                      \
+                TDGS_CALL(STEP, CL, RE, "3", TDGS_SET1, DF1, LM,                                                      \
                           TDGS_READ(RC, "v[40:43]", "v[44:47]", "v[48:49]", "v48", "192", "208", "224"))      \
     "v_add_u32 v39, 0xc0, v39\n"                                                                              \
     "s_add_u32 %[idx], %[idx], 4\n"                                                                           \
@@ -1669,19 +1681,19 @@ __device__ __forceinline__ void blend_batch(uint32_t lds_addr, int32_t idx0, int
 #define TDGS_IN(P, I)                                                                                    \
     [uu##P] "v"(px[I].uu), [vv##P] "v"(px[I].vv), [uv##P] "v"(px[I].uv), [cu##P] "v"(px[I].cu), [cv##P] "v"(px[I].cv)
 #define TDGS_COMMON_IN                                                                              \
-    [addr] "v"(lds_addr), [i0] "s"(idx0), [iend] "s"(idx_end), [c5] "v"(c5), [cut] "s"(e_exact),     \
-        [maxa] "s"(max_alpha), [minT] "s"(min_T)
+    [addr] "v"(lds_addr), [i0] "s"(idx0), [iend] "s"(idx_end), [c5] "v"(c5), [cut] "s"(cut),         \
+        [mina] "s"(min_alpha), [maxa] "s"(max_alpha), [minT] "s"(min_T)
 #define TDGS_CLOBBERS                                                                                       \
     "v38", "v39", "v40", "v41", "v42", "v43", "v44", "v45", "v46", "v47", "v48", "v49", "v50", "v51", "v52", \
         "v53", "v54", "v55", "v56", "v57", "v58", "v59", "v60", "v61", "v62", "v63", "vcc", "scc", "memory"
-#define TDGS_BLEND1(RC, DF0, DF1, LM, MORE)                                                                           \
-    asm volatile(TDGS_LOOP(TDGS_STEP1, "s_mov_b64 exec, %[act0]\n", RC, DF0, DF1, LM) TDGS_STOP1("0")           \
+#define TDGS_BLEND1(CL, RE, RC, DF0, DF1, LM, MORE)                                                                           \
+    asm volatile(TDGS_LOOP(TDGS_STEP1, "s_mov_b64 exec, %[act0]\n", CL, RE, RC, DF0, DF1, LM) TDGS_STOP1("0")           \
                      TDGS_STOP1("1") TDGS_STOP1("2") TDGS_STOP1("3") TDGS_TAIL                                  \
                  : [ent] "=&s"(ent), [idx] "=&s"(idx), TDGS_OUT(0, 0) MORE(0, 0)                                           \
                  : TDGS_COMMON_IN, TDGS_IN(0, 0)                                                                \
                  : TDGS_CLOBBERS)
-#define TDGS_BLEND2(RC, DF0, DF1, LM, MORE)                                                                           \
-    asm volatile(TDGS_LOOP(TDGS_STEP2, "", RC, DF0, DF1, LM) TDGS_STOP2("0", "0") TDGS_STOP2("1", "0")          \
+#define TDGS_BLEND2(CL, RE, RC, DF0, DF1, LM, MORE)                                                                           \
+    asm volatile(TDGS_LOOP(TDGS_STEP2, "", CL, RE, RC, DF0, DF1, LM) TDGS_STOP2("0", "0") TDGS_STOP2("1", "0")          \
                      TDGS_STOP2("2", "0") TDGS_STOP2("3", "0") TDGS_STOP2("0", "1") TDGS_STOP2("1", "1")        \
                          TDGS_STOP2("2", "1") TDGS_STOP2("3", "1") TDGS_TAIL                                    \
                  : [ent] "=&s"(ent), [idx] "=&s"(idx), [lv] "=&s"(lv), TDGS_OUT(0, 0) MORE(0, 0), TDGS_OUT(1, 1) MORE(1, 1)           \
@@ -1696,12 +1708,23 @@ __device__ __forceinline__ void blend_batch(uint32_t lds_addr, int32_t idx0, int
 // the last contributing index is tracked only when it is an output
 #define TDGS_LAST_ON(P, K) "v_add_u32_e64 %[L" P "], %[idx], " K "\n"
 #define TDGS_LAST_OFF(P, K) ""
+// (two compares: exponents above 88 or NaN to 88, lanes whose alpha falls short of min_alpha out of exec)
+#define TDGS_CLAMP(E) "v_min_f32 " E ", 0x42b00000, " E "\n"
+#define TDGS_REACH                        \
+    "v_cmp_ngt_f32 vcc, %[mina], v63\n"  \
+    "s_and_b64 exec, exec, vcc\n"
+#define TDGS_NO_CLAMP(E) ""
 #define TDGS_BLEND(F)                                                                           \
     do {                                                                                        \
-        if constexpr (DEPTH && LAST) F(TDGS_READ_BD, TDGS_DEPTH_ON0, TDGS_DEPTH_ON1, TDGS_LAST_ON, TDGS_OUT_DL);   \
-        else if constexpr (DEPTH) F(TDGS_READ_BD, TDGS_DEPTH_ON0, TDGS_DEPTH_ON1, TDGS_LAST_OFF, TDGS_OUT_D);     \
-        else if constexpr (LAST) F(TDGS_READ_B, TDGS_DEPTH_OFF, TDGS_DEPTH_OFF, TDGS_LAST_ON, TDGS_OUT_L);        \
-        else F(TDGS_READ_B, TDGS_DEPTH_OFF, TDGS_DEPTH_OFF, TDGS_LAST_OFF, TDGS_OUT_NONE);                           \
+        if constexpr (EXACT) TDGS_BLEND_OUT(F, TDGS_NO_CLAMP, "");                              \
+        else TDGS_BLEND_OUT(F, TDGS_CLAMP, TDGS_REACH);                                         \
+    } while (0)
+#define TDGS_BLEND_OUT(F, CL, RE)                                                               \
+    do {                                                                                        \
+        if constexpr (DEPTH && LAST) F(CL, RE, TDGS_READ_BD, TDGS_DEPTH_ON0, TDGS_DEPTH_ON1, TDGS_LAST_ON, TDGS_OUT_DL);   \
+        else if constexpr (DEPTH) F(CL, RE, TDGS_READ_BD, TDGS_DEPTH_ON0, TDGS_DEPTH_ON1, TDGS_LAST_OFF, TDGS_OUT_D);     \
+        else if constexpr (LAST) F(CL, RE, TDGS_READ_B, TDGS_DEPTH_OFF, TDGS_DEPTH_OFF, TDGS_LAST_ON, TDGS_OUT_L);        \
+        else F(CL, RE, TDGS_READ_B, TDGS_DEPTH_OFF, TDGS_DEPTH_OFF, TDGS_LAST_OFF, TDGS_OUT_NONE);                           \
     } while (0)
     if constexpr (PX == 1) {
         (void)lv;
@@ -1739,6 +1762,10 @@ __device__ __forceinline__ void blend_batch(uint32_t lds_addr, int32_t idx0, int
 #undef TDGS_LAST_ON
 #undef TDGS_LAST_OFF
 #undef TDGS_BLEND
+#undef TDGS_BLEND_OUT
+#undef TDGS_CLAMP
+#undef TDGS_NO_CLAMP
+#undef TDGS_REACH
 }
 
 // One workgroup per tile, one thread per PX pixels (tile_pixel; wavefront w takes pixels 64 PX w + 64 k +
@@ -1747,9 +1774,9 @@ __device__ __forceinline__ void blend_batch(uint32_t lds_addr, int32_t idx0, int
 // lane reads the same record (broadcast). A wavefront skips an entry for a block when no pixel it
 // still blends can reach min_alpha, leaves the batch when all its pixels
 // are done, and the tile stops loading batches once every pixel is done. The steps of a batch
-// run in blend_batch, except for the counting replay (COUNT) and for batches whose live
-// exponents may leave [-80, 88] or hold NaN parameters (`checked`), which take the loop below
-// with exp_f's range handling.
+// run in blend_batch, except for the counting replay (COUNT) and for thresholds that let live
+// exponents fall below -87 or max_alpha pass exp_f(88) (kStepsCompiled), which take the loop below with exp_f's
+// range handling.
 //
 // Two pixels per lane halve the wavefronts, and a wavefront's walk gets longer: it pays only where
 // many rounds of workgroups follow each other (the last one's length no longer counts), and there
@@ -1843,11 +1870,11 @@ __global__ __launch_bounds__(1024 / PX) __attribute__((amdgpu_waves_per_eu(PX ==
                 odd = odd || !plain;
             }
         }
-        // A live exponent lies in [e_exact, log a + 65]; unless e_exact < -80 or a record of the
-        // batch is odd, that is inside [-87, 88], where exp_f is its polynomial core.
-        const bool checked = __syncthreads_or(odd) || a.checked;
+        // Without an odd record a live exponent lies in [cut, log a + 65], inside [-87, 88], where
+        // exp_f is its polynomial core.
+        const bool any_odd = __syncthreads_or(odd);
         const int nb = (int)((end - base) < NB ? (end - base) : NB);
-        if (!COUNT && !checked) {
+        if (!COUNT && a.steps != kStepsCompiled) {
             uint64_t act[PX], any = 0;
 #pragma unroll
             for (int k = 0; k < PX; ++k) {
@@ -1856,8 +1883,11 @@ __global__ __launch_bounds__(1024 / PX) __attribute__((amdgpu_waves_per_eu(PX ==
             }
             if (any != 0) {
                 const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) BlendRec*)s_rec;
-                blend_batch<DEPTH, LAST, PX>(lds, (int32_t)(base + 1), (int32_t)(base + nb + 1), a.e_exact,
-                                             a.max_alpha, a.min_T, px, act);
+                const int32_t i0 = (int32_t)(base + 1), i1 = (int32_t)(base + nb + 1);
+                if (a.steps == kStepsExact && !any_odd)
+                    blend_batch<true, DEPTH, LAST, PX>(lds, i0, i1, a.e_exact, a.min_alpha, a.max_alpha, a.min_T, px, act);
+                else
+                    blend_batch<false, DEPTH, LAST, PX>(lds, i0, i1, a.e_cut, a.min_alpha, a.max_alpha, a.min_T, px, act);
 #pragma unroll
                 for (int k = 0; k < PX; ++k) done[k] = ((act[k] >> __lane_id()) & 1ull) == 0;
             }
@@ -1876,8 +1906,7 @@ __global__ __launch_bounds__(1024 / PX) __attribute__((amdgpu_waves_per_eu(PX ==
                 if (!wave_any(live)) continue;
                 // exp_f(e) for the live lanes: the polynomial core unless a live lane is outside
                 // [-87, 88] or NaN (the other lanes' values are not used)
-                const float ex = (checked && wave_any(live && !(e >= -87.0f && e <= 88.0f))) ? exp_f_sel(e)
-                                                                                            : exp_f_core(e);
+                const float ex = wave_any(live && !(e >= -87.0f && e <= 88.0f)) ? exp_f_sel(e) : exp_f_core(e);
                 // min(ex, max_alpha); equal to the select ex < max_alpha ? ex : max_alpha for a
                 // non-NaN max_alpha, NaN ex included
                 const float alpha = __builtin_fminf(ex, a.max_alpha);
@@ -1977,7 +2006,8 @@ static int launch_render_tiles(hipStream_t s, const tdgs_camera* cam, const tdgs
     a.bg0 = o->background[0]; a.bg1 = o->background[1]; a.bg2 = o->background[2];
     a.min_alpha = o->min_alpha; a.max_alpha = o->max_alpha; a.min_T = o->min_transmittance;
     a.e_cut = exponent_cut(o->min_alpha);
-    a.checked = !exact_exponent_cut(o->min_alpha, o->max_alpha, &a.e_exact);
+    a.steps = exact_exponent_cut(o->min_alpha, o->max_alpha, &a.e_exact) ? kStepsExact : kStepsGeneral;
+    if (!(a.e_cut >= -87.0f) || !(o->max_alpha <= 1e38f)) a.steps = kStepsCompiled;
     a.m = m; a.tiles_end = tiles_end; a.sorted_f = sorted_f; a.f2d = f2d; a.depths = depths;
     a.rgb = out->rgb; a.T = out->T; a.depth = out->depth; a.last = out->last;
     a.evaluations = evaluations;
