@@ -93,7 +93,7 @@ def copy_calibration():
 # rocprofv3 kernel names -> the counter summary's keys (the first match wins; the blend is the
 # timed render's variant, without last-contributor output)
 TRAFFIC_KERNELS = [
-    ("k_render_tiles<true, false, false, false>", "blend"),
+    ("k_render_tiles<true, false, false, false", "blend"),   # (of one or two pixels per lane)
     ("k_backward_blend<", "backward_blend"),
     ("k_project<", "project"),
     ("k_keep_counts", "keep_counts"),
@@ -102,19 +102,22 @@ TRAFFIC_KERNELS = [
     ("k_emit_scatter<", "coarse_sort_scatter"),
     ("k_backward_project<false>", "backward_project"),
     ("k_backward_project<true>", "backward_project_adam"),
-    ("k_rs_scatter_grouped<unsigned int>", "depth_sort_scatter"),
+    ("k_rs_scatter_grouped<unsigned int>", "depth_sort_scatter"),   # (to 2.1M Gaussians)
     ("k_rs_count_grouped<unsigned int>", "depth_sort_count"),
+    ("k_rs_scatter<unsigned int>", "depth_sort_scatter"),
+    ("k_rs_count<unsigned int>", "depth_sort_count"),
+    ("k_rs_scan_rows", "depth_sort_scan_rows"),
     ("k_ds_count", "depth_sort_bucket_count"),
     ("k_ds_scatter", "depth_sort_bucket_scatter"),
     ("k_ds_buckets", "depth_sort_buckets"),
     ("k_ssim_forward", "loss_ssim_forward"),
     ("k_ssim_backward", "loss_ssim_backward"),
-    ("k_bin_tiles<3, false>", "bin_count"),
-    ("k_bin_tiles<3, true>", "bin_write"),
-    ("k_bin_tiles<4, false>", "bin_count_16x"),
-    ("k_bin_tiles<4, true>", "bin_write_16x"),
+    ("k_bin_tiles<3, false, false>", "bin_count"),
+    ("k_bin_tiles<3, true, false>", "bin_write"),
+    ("k_bin_tiles<4, false, false>", "bin_count_16x"),
+    ("k_bin_tiles<4, true, false>", "bin_write_16x"),
     ("k_bin_scan", "bin_scan"),
-    ("k_scan_apply<tdgs::SortedTileBlockCounts", "count_scan_apply"),
+    ("k_scan_apply<true, tdgs::SortedBlockCounts", "count_scan_apply"),
 ]
 
 
@@ -645,7 +648,8 @@ MEASURED_KERNELS = {
     "K2_scan_keys": [("count_scan_apply", 1), ("emit_count", 1)],
     "K3_K4_sort_ranges": [("depth_sort_bucket_count", 1), ("depth_sort_bucket_scatter", 1), ("depth_sort_buckets", 1),
                           ("coarse_sort_scatter", 1), ("bin_count", 1), ("bin_scan", 1), ("bin_write", 1)],
-    "K3_K4_sort_ranges_radix": [("depth_sort_count", 4), ("depth_sort_scatter", 4), ("coarse_sort_scatter", 1),
+    "K3_K4_sort_ranges_radix": [("depth_sort_count", 4), ("depth_sort_scan_rows", 4), ("depth_sort_scatter", 4),
+                                ("coarse_sort_scatter", 1),
                                 ("bin_count", 1), ("bin_scan", 1), ("bin_write", 1)],
     "K5_blend": [("blend", 1)],
     "K6_backward_blend": [("backward_blend", 1)],

@@ -2017,13 +2017,13 @@ static int launch_render_tiles(hipStream_t s, const tdgs_camera* cam, const tdgs
     a.mon_host = mon_host;
     const int nt = t->tile_width * t->tile_height;
     const dim3 grid(t->nb_tiles_x, t->nb_tiles_y);
-    // + the padding after a batch and the record blend_batch reads past its last group of four
-    // Two pixels per lane where that leaves at least three rounds of the chip's 8192 wavefronts: see
-    // k_render_tiles.
+    // Two pixels per lane where that leaves at least four rounds of the 6144 wavefronts (6 per SIMD)
+    // that run at once: see k_render_tiles.
     const int64_t waves2 = (int64_t)t->nb_tiles_x * t->nb_tiles_y * (nt / (2 * kWave));
     const bool two = t->tile_width % 8 == 0 && t->tile_height % 8 == 0 && nt % (2 * kWave) == 0 &&
                      waves2 >= kBlendWaves2 && !evaluations;
     a.batch = two ? kBlendBatch2 : nt;
+    // + the padding after a batch and the record blend_batch reads past its last group of four
     const size_t lds = (size_t)(a.batch + 4) * sizeof(BlendRec);
     if (evaluations) {
         k_render_tiles<false, false, true><<<grid, nt, lds, s>>>(a);
