@@ -254,7 +254,7 @@ def test_render_tiny_min_alpha_takes_range_checked_path(gpu, oracle):
 
 def test_render_only_huge_opacities_take_range_checked_path(gpu, oracle):
     """Render-only opacities above 1e38 make live exponents exceed 88 in their batches, which
-    then use the range-checked loop; the other batches the fast steps."""
+    then take the steps that clamp them; the other batches the fast ones."""
     from tdgs_amd import ply
     w = synthetic.config(0, n=3000)
     ro = ply.to_render_only(w.gaussians)
@@ -357,8 +357,8 @@ def test_render_list_lengths_at_batch_ends_of_large_images(gpu, oracle, k):
     (0.5, 0.3), (1.9e-35, 0.99), (1e-36, 0.99), (0.0, 0.99)])
 @pytest.mark.parametrize("w,h", [(256, 256), (2048, 1600)])
 def test_render_alpha_thresholds_bit_exact(gpu, oracle, min_alpha, max_alpha, w, h):
-    """The exponent that stands for min_alpha, over the range of thresholds it is used for and outside it
-    (above 0.9, below exp(-80), above max_alpha, none), where the compares of alpha remain."""
+    """The exponent that stands for min_alpha, over the range of thresholds it is used for (above max_alpha
+    included: none is reached) and outside it (above 0.9, below exp(-80), none), where alpha is compared."""
     wl = synthetic.config(0, n=300)
     wl.gaussians.means_opacity[:, 3] = np.random.default_rng(1).normal(0.0, 3.0, 300)
     cam = host.look_at_camera(w, h, 60.0, (0.0, 0.0, -4.0))

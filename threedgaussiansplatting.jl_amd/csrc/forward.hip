@@ -1170,9 +1170,10 @@ __global__ __launch_bounds__(1024) void k_bin_tiles(BinArgs a) {
             // tile-major walk from 16 hits per 64 candidates alone measured 45 -> 49 us.)
             // It also takes what the candidate-major loop does not: a frame whose keys do not fit (an index
             // past a.cap - 1 is clamped; the frame is thrown away) and lists past 32-bit byte offsets.
-            // (752M keys, 3.0 GB, at 3840 x 2160: 4.1 TB/s of writes, and no faster with half the
+            // (752M keys, 3.0 GB, at 3840 x 2160: 4.2 TB/s of writes, and no faster with half the
             // instructions, with full aligned 1 KB stores through an LDS ring, or with chunks twice as
-            // long; non-temporal stores double the time. Memory it is.)
+            // long; non-temporal stores double the time. A fill reaches 6.9: the runs of ~4 KB to scattered
+            // places bound it.)
             const bool fits = WRITE && __ballot(lane < 16 && start + seg_hits > min(a.cap, 1 << 30)) == 0;
             if (WRITE && (!fits || (wave_hits >= 4 * nk && wave_hits >= 16 * 256))) {
                 const int row0 = 16 + __builtin_amdgcn_readfirstlane(ly0);
