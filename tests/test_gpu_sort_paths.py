@@ -128,3 +128,28 @@ def test_depth_presort_bucket_past_capacity(gpu, oracle):
         if device_counts:
             assert buf.frame_counts()[3] == abi.TDGS_FRAME_OK
         _assert_forward_equal(r, out, buf)
+
+
+@pytest.mark.parametrize("n", [1, 5000, 100_000])
+def test_sort_pairs_in_scratch_without_group_sums(gpu, n):
+    """Scratch of the size a sort cannot do without (what tdgs_sort_pairs_temp_bytes asked for before the
+    grouped tables came in) is accepted and sorts the same; less is refused."""
+    lib, dev = gpu.lib(), torch.device("cuda", 0)
+    rng = np.random.default_rng(n)
+    keys = rng.integers(0, 1 << 20, n).astype(np.int64)
+    k, v = torch.from_numpy(keys).to(dev), torch.arange(n, dtype=torch.int32, device=dev)
+    groups = -(-(-(-n // 4096)) // 16)
+    base = int(lib.tdgs_sort_pairs_temp_bytes(n, 45)) - 8 * groups * 256 * 4
+    temp = torch.empty(base, dtype=torch.uint8, device=dev)
+    ko, vo = torch.empty_like(k), torch.empty_like(v)
+
+    def sort(size):
+        return lib.tdgs_sort_pairs(gpu.dptr(temp), size, gpu.dptr(k), gpu.dptr(ko), gpu.dptr(v), gpu.dptr(vo), n, 45,
+                                   gpu.stream_ptr(0))
+
+    gpu.check(sort(base))
+    order = np.argsort(keys, kind="stable")
+    np.testing.assert_array_equal(vo.cpu().numpy(), order)
+    np.testing.assert_array_equal(ko.cpu().numpy(), keys[order])
+    with pytest.raises(gpu.TdgsError, match="scratch too small"):
+        gpu.check(sort(base - 1))

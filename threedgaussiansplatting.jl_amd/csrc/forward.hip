@@ -2502,11 +2502,16 @@ static int64_t sort_pairs_group_words(int64_t n) {
     return radix_group_words<uint64_t>(n < most ? n : most, 0, 64);
 }
 
+// The scratch a sort cannot do without; with the group sums besides, sorts of few pairs take two launches a
+// pass instead of three.
+static size_t sort_pairs_base_bytes(int64_t n) {
+    return align_up((size_t)n * sizeof(int64_t)) + align_up((size_t)n * sizeof(int32_t)) + radix_temp_bytes(n);
+}
+
 size_t tdgs_sort_pairs_temp_bytes(int32_t n, int32_t end_bit) {
     (void)end_bit;
     const int64_t nn = n > 0 ? n : 1;
-    return align_up((size_t)nn * sizeof(int64_t)) + align_up((size_t)nn * sizeof(int32_t)) +
-           align_up(radix_temp_bytes(nn)) + (size_t)sort_pairs_group_words(nn) * sizeof(uint32_t);
+    return sort_pairs_base_bytes(nn) + (size_t)sort_pairs_group_words(nn) * sizeof(uint32_t);
 }
 
 int tdgs_sort_pairs(void* temp, size_t temp_bytes, const int64_t* keys_in, int64_t* keys_out,
@@ -2516,13 +2521,13 @@ int tdgs_sort_pairs(void* temp, size_t temp_bytes, const int64_t* keys_in, int64
     if (n == 0) return TDGS_OK;
     TDGS_REQUIRE(keys_in && keys_out && values_in && values_out && temp, "null arrays");
     TDGS_REQUIRE(keys_in != keys_out && values_in != values_out, "sort_pairs is not in place");
-    TDGS_REQUIRE(temp_bytes >= tdgs_sort_pairs_temp_bytes(n, end_bit), "sort scratch too small");
+    TDGS_REQUIRE(temp_bytes >= sort_pairs_base_bytes(n), "sort scratch too small");
     Arena ar(temp, temp_bytes);
     uint64_t* alt_k = ar.take<uint64_t>(n);
     int32_t* alt_v = ar.take<int32_t>(n);
     const size_t rb = radix_temp_bytes(n);
     void* rtemp = ar.take<char>((int64_t)rb);
-    uint32_t* grp = nullptr;
+    uint32_t* grp = nullptr;   // (null, also where the scratch ends before them: without grouped tables)
     int64_t words = 0;
     if (radix_tiles<uint64_t>(n) <= RsTile<uint64_t>::kGroupedTiles) {
         words = radix_group_words<uint64_t>(n, 0, end_bit);
