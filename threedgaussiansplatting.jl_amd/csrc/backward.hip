@@ -129,6 +129,8 @@ struct BackBlendArgs {
 // nine), so they also must fit back_fits' rounds. 24x24 tiles at PX = 4, 2, 1: 720x720 (900 tiles, 512 of five
 // wavefronts at a time) 111.5, 86.7, 98.6 (R), 183.5, 234.2, 243.1 (B), 136.8, 186.1, 200.3 (D); 660x600 (700
 // tiles) 127.7, 76.6, 74.4; 186.1, 186.8, 201.2; 132.2, 139.6, 162.1.
+// (Close to the line the long lists lose most there: 48x16, 979x546, 735 tiles of six wavefronts at PX = 2, 178 and 154 us
+// (B, D) where PX = 4 takes 158 and 119; R 81 against 90.)
 // Tiles of at most 64 PX / 2 pixels would leave half the lanes off (8 x 8 tiles, 800x800: 67.8, 65.0, 58.3; 210.3,
 // 201.7, 178.4; 257.7, 268.0, 250.8).
 constexpr int64_t kBackWaves1 = 6144, kBackWaves2 = 9216;   // blocks up to which PX is 1, 2
